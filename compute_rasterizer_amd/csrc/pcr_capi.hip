@@ -276,6 +276,8 @@ int pcr_cloud_upload_batched(pcr_ctx* ctx, const pcr_batch* batches, uint32_t nb
     PCR_HIP_OR(hipMemcpy(c->d_rgba, rgba, npoints * 4, hipMemcpyHostToDevice), drop());
     PCR_HIP_OR(hipStreamSynchronize(ctx->stream), drop());
     c->h_batches.assign(batches, batches + nb);
+    rc = cloud_build_groups(ctx, c);
+    if (rc) { drop(); return rc; }
     *out = c;
     return PCR_OK;
 }

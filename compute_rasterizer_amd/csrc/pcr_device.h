@@ -299,9 +299,10 @@ __device__ __forceinline__ void project_interior(const Proj& p, float x, float y
 //     rectangle with its 1-pixel margin (the same holds for y with H).
 __device__ inline bool screen_rect(const float* __restrict__ t, const float mn[3], const float mx[3], int w, int h,
                                    int& x0, int& y0, int& x1, int& y1, bool* interior = nullptr,
-                                   float* wlo = nullptr) {
+                                   float* wlo = nullptr, float* wnear = nullptr) {
     if (interior) *interior = false;
     if (wlo) *wlo = 0.0f;
+    if (wnear) *wnear = 0.0f;
     const int c = (int)(__lane_id() & 7u);
     const float x = (c & 1) ? mx[0] : mn[0], y = (c & 2) ? mx[1] : mn[1], z = (c & 4) ? mx[2] : mn[2];
     const float px = fma_(t[8], z, fma_(t[4], y, fma_(t[0], x, t[12])));
@@ -342,8 +343,97 @@ __device__ inline bool screen_rect(const float* __restrict__ t, const float mn[3
             if (pwmin >= fmaxf((float)w, (float)h) * 0x1p-21f * (fmaxf(ex, ey) + ew))
                 *wlo = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(pwmin - 0x1p-18f * ew)));
         }
+        // the same depth for a box that need not lie inside the image
+        if (wnear && __ballot(!ok) == 0ull) {
+            float pwmin = pw;
+#pragma unroll
+            for (int m = 1; m < 8; m <<= 1) pwmin = fminf(pwmin, __shfl_xor(pwmin, m));
+            if (pwmin >= fmaxf((float)w, (float)h) * 0x1p-21f * (fmaxf(ex, ey) + ew))
+                *wnear = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(pwmin - 0x1p-18f * ew)));
+        }
     }
     return x1 >= x0 && y1 >= y0;
+}
+
+// ------------------------------------------------------------ group bounds
+// group_rect()'s bounds for a batch with a positive `wlo` or `wnear` from
+// screen_rect().
+struct GroupSlack {
+    float px, w;
+};
+__device__ __forceinline__ GroupSlack group_slack(const float* __restrict__ t, const float mn[3], const float mx[3],
+                                                  int w, int h, float wlo) {
+    const float ax = fmaxf(fabsf(mn[0]), fabsf(mx[0])), ay = fmaxf(fabsf(mn[1]), fabsf(mx[1])),
+                az = fmaxf(fabsf(mn[2]), fabsf(mx[2]));
+    const float ex = fabsf(t[12]) + fabsf(t[0]) * ax + fabsf(t[4]) * ay + fabsf(t[8]) * az;
+    const float ey = fabsf(t[13]) + fabsf(t[1]) * ax + fabsf(t[5]) * ay + fabsf(t[9]) * az;
+    const float ew = fabsf(t[15]) + fabsf(t[3]) * ax + fabsf(t[7]) * ay + fabsf(t[11]) * az;
+    const float side = fmaxf((float)w, (float)h), spread = side * 0x1p-21f * (fmaxf(ex, ey) + ew);
+    GroupSlack s;
+    s.px = spread / wlo + side * 0x1p-19f;
+    s.w = 0x1p-19f * ew;
+    return s;
+}
+
+// The pixels that the points of one group can land in, and a depth none of
+// them undercuts. `box` holds the smallest and the largest coarse coordinate
+// of the group on each axis, and a decoded position lies between the decoded
+// bounds exactly: a rounded fma keeps the order of its operands, and at the
+// 20- and 30-bit levels float(X) lies between l * 2^20 and (l + 1) * 2^20.
+//
+// With the box's centre c and half edges e, a point p of it projects to
+//   n(p) - n(c) = (dX - n(c) dW) / (w(c) + dW),  dX - n(c) dW = sum_a d_a (tx_a - n(c) tw_a),
+// so |n(p) - n(c)| <= sum_a e_a |tx_a - n(c) tw_a| / (w(c) - sum_a e_a |tw_a|).
+//
+// Rounding, with u = 2^-24, R = (max(ex, ey) + ew) / (smallest corner depth of
+// the batch), M = max(1, |n|) and sum e |tw| at most half of w(c) (else `wild`):
+//   - n(c): 3 roundings a row, 1 ulp (2u) of v_rcp_f32, the product: M(3uR + 3u);
+//   - the centre's own rounding shifts the box by u of its coordinates: M uR;
+//   - the radius: n's error times sum e |tw| / (w - ..) <= 1, 5u of its terms,
+//     the divisor's M(3uR + 5u), the reciprocal and product 3u: M(6uR + 16u);
+//   - a point's computed coordinate (3 roundings a row, the division, the
+//     scaling): 3uR + 5u;
+//   - the conversion to pixels: 8u M of NDC.
+// Half the image times the sum is W*u*M (6.5 R + 16); slack_px is W*u (8 R + 32)
+// without M, and the 2^-16 * ew condition keeps the error of R below 3%.
+// Depths differ by at most 12u*ew, below slack_w = 32u*ew.
+struct GroupRect {
+    int x0, y0, x1, y1;   // clamped to the image; empty when x1 < x0 or y1 < y0
+    float w;              // depth
+    bool wild;            // no bound (a box that reaches the eye or lies far outside the image)
+};
+__device__ __forceinline__ GroupRect group_rect(uint2 box, int level, const Decode& d, const float* __restrict__ t,
+                                                int w, int h, float slack_px, float slack_w) {
+    const float step = level <= 1 ? 1048576.0f : 1.0f, open = level <= 1 ? 1.0f : 0.0f;
+    float c[3], e[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float l = fma_((float)((box.x >> (10 * a)) & 1023u) * step, d.scale[a], d.mn[a]);
+        const float u = fma_(((float)((box.y >> (10 * a)) & 1023u) + open) * step, d.scale[a], d.mn[a]);
+        c[a] = 0.5f * (l + u);
+        e[a] = 0.5f * fabsf(u - l);
+    }
+    const float px = fma_(t[8], c[2], fma_(t[4], c[1], fma_(t[0], c[0], t[12])));
+    const float py = fma_(t[9], c[2], fma_(t[5], c[1], fma_(t[1], c[0], t[13])));
+    const float pw = fma_(t[11], c[2], fma_(t[7], c[1], fma_(t[3], c[0], t[15])));
+    const float ew = fma_(e[2], fabsf(t[11]), fma_(e[1], fabsf(t[7]), e[0] * fabsf(t[3])));
+    const float iv = __builtin_amdgcn_rcpf(pw), lw = pw - ew, il = __builtin_amdgcn_rcpf(lw);
+    const float nx = px * iv, ny = py * iv;
+    const float rx = fma_(e[2], fabsf(fma_(-nx, t[11], t[8])),
+                          fma_(e[1], fabsf(fma_(-nx, t[7], t[4])), e[0] * fabsf(fma_(-nx, t[3], t[0]))));
+    const float ry = fma_(e[2], fabsf(fma_(-ny, t[11], t[9])),
+                          fma_(e[1], fabsf(fma_(-ny, t[7], t[5])), e[0] * fabsf(fma_(-ny, t[3], t[1]))));
+    const float fw = 0.5f * (float)w, fh = 0.5f * (float)h;
+    const float m = fmaxf(fmaxf(fabsf(nx) + rx * il, fabsf(ny) + ry * il), 1.0f), s = slack_px * m;
+    const float cx = fma_(nx, fw, fw), cy = fma_(ny, fh, fh), dx = fma_(rx * il, fw, s), dy = fma_(ry * il, fh, s);
+    GroupRect g;
+    g.wild = !(m <= 64.0f && ew <= 0.5f * pw);
+    g.x0 = max((int)floorf(cx - dx), 0);
+    g.y0 = max((int)floorf(cy - dy), 0);
+    g.x1 = min((int)floorf(cx + dx), w - 1);
+    g.y1 = min((int)floorf(cy + dy), h - 1);
+    g.w = lw - slack_w;
+    return g;
 }
 
 // A batch's screen rectangle for one view, as screen_rect() reports it.

@@ -284,6 +284,8 @@ int pcr_cloud_from_las(pcr_ctx* ctx, const pcr_las_file* files, int nfiles, uint
             c->aabb_min[a] = h.min[a] < c->aabb_min[a] ? h.min[a] : c->aabb_min[a];
             c->aabb_max[a] = h.max[a] > c->aabb_max[a] ? h.max[a] : c->aabb_max[a];
         }
+    rc = cloud_build_groups(ctx, c);
+    if (rc) { cloud_free(c); delete c; return rc; }
     if (first_batch) memcpy(first_batch, fb.data(), sizeof(uint32_t) * (nfiles + 1));
     *out = c;
     return PCR_OK;
@@ -339,6 +341,8 @@ int pcr_cloud_from_potree(pcr_ctx* ctx, const pcr_potree_info* info, const void*
             c->aabb_min[a] = h.min[a] < c->aabb_min[a] ? h.min[a] : c->aabb_min[a];
             c->aabb_max[a] = h.max[a] > c->aabb_max[a] ? h.max[a] : c->aabb_max[a];
         }
+    rc = cloud_build_groups(ctx, c);
+    if (rc) { cloud_free(c); delete c; return rc; }
     *out = c;
     return PCR_OK;
 }

@@ -8,10 +8,22 @@
 
 namespace pcr {
 
+// Points per group: 64 words of the coarse plane, counted from the 16-byte
+// aligned word at or below the batch's first point.
+constexpr uint32_t kGroupPoints = 64;
+__host__ __device__ inline uint32_t groups_of(uint32_t first, uint32_t n) {
+    return (uint32_t)(((uint64_t)n + (first & 3u) + kGroupPoints - 1) / kGroupPoints);
+}
+
+// The select stage lists the drawn batches in kSlices slices of the view
+// depth, the nearest first: slice k of a cloud of nb batches starts at
+// list[k * nb].
+constexpr uint32_t kSlices = 8;
+
 // Per-frame counters in device memory, zeroed by a kernel at frame start
 // (a kernel rather than a memset so that the frame can be graph-captured).
 struct FrameState {
-    uint32_t list_count;        // batches appended by the select stage
+    uint32_t slice_count[kSlices];   // batches appended by the select stage, by slice
     uint32_t queue_head;        // work items taken by the raster stage (hqs: pass 1)
     uint32_t queue_head2;       // hqs: work items taken by pass 2
     uint32_t level_count[5];
@@ -19,7 +31,7 @@ struct FrameState {
     unsigned long long points_drawn;
     unsigned long long plane_bytes;
     uint32_t occluded_batches;          // batch draws skipped by the occlusion test (rect_open)
-    unsigned long long occluded_points; // their points
+    unsigned long long occluded_points; // their points, and those of the skipped groups of others
     unsigned long long occluded_bytes;  // the plane (hqs pass 2: and colour) bytes they did not read
     unsigned long long atomics;         // 64-bit framebuffer atomics issued (LAS, LAS2, NODES)
     unsigned long long pixels_visible;  // pixels the index resolve found covered
@@ -83,7 +95,10 @@ struct pcr_cloud {
     uint4* d_points16 = nullptr;          // x, y, z (float bits), rgba
     uint64_t points16_len = 0;
     uint8_t* d_levels = nullptr;          // per-batch level of the last frame (255 = not drawn)
-    uint32_t* d_list = nullptr;           // compacted list of drawn batches
+    uint32_t* d_list = nullptr;           // compacted lists of drawn batches, list_slices * num_batches entries
+    uint32_t list_slices = 1;             // 1 or kSlices
+    uint2* d_gbox = nullptr;              // coarse-plane bounds of each batch's groups (null: none)
+    uint32_t* d_gbase = nullptr;          // per batch: its first group in d_gbox
     int num_levels = 0;                   // octree depth + 1 (LOD clouds)
     float aabb_min[3] = {0, 0, 0};
     float aabb_max[3] = {0, 0, 0};
@@ -177,6 +192,9 @@ int generate_points(pcr_ctx* ctx, const pcr_gen_cfg* cfg, float* xyz, uint32_t* 
 int build_cloud_device(pcr_ctx* ctx, const float* xyz, const uint32_t* rgba, uint64_t n,
                        const pcr_build_opts* opts, pcr_cloud** out);
 int cloud_alloc_batched(pcr_ctx* ctx, uint32_t nb, uint64_t npoints, pcr_cloud* c);
+// Group bounds of a finished batched cloud (headers in h_batches, planes on the
+// device). Without the memory for them the cloud has none.
+int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c);
 int device_aabb(pcr_ctx* ctx, const float* xyz, uint64_t n, float mn[3], float mx[3]);
 int build_octree_device(pcr_ctx* ctx, const float* xyz, const uint32_t* rgba, uint64_t n, const pcr_octree_opts* o,
                         pcr_cloud** out);

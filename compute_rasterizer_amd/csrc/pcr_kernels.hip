@@ -63,7 +63,8 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
 // A frame's counters are zeroed by the select launch of the frame before it
 // (k_select resets the other of the context's two frame states).
 __device__ __forceinline__ void frame_reset(FrameState* st) {
-    st->list_count = 0; st->queue_head = 0; st->queue_head2 = 0; st->culled = 0;
+    for (uint32_t k = 0; k < kSlices; k++) st->slice_count[k] = 0;
+    st->queue_head = 0; st->queue_head2 = 0; st->culled = 0;
     for (int i = 0; i < 5; i++) st->level_count[i] = 0;
     st->points_drawn = 0; st->plane_bytes = 0;
     st->occluded_batches = 0; st->occluded_points = 0; st->occluded_bytes = 0; st->atomics = 0;
@@ -124,6 +125,23 @@ constexpr int kSelectBlock = 1024;
 // stores over the whole grid; the raster runs after it on the stream) and
 // resets the other frame state for the next frame, so a frame needs no
 // launch before its select.
+//
+// The list is kept in slices of the batches' nearest view depth, equal steps
+// of its logarithm, the nearest first (SliceRule): the raster draws the slices
+// in order, so that the depths a far batch is tested against are already
+// there.
+struct SliceRule {
+    float inv_near, scale;   // slice = log2(w * inv_near) * scale; scale 0: one slice
+};
+__device__ __forceinline__ uint32_t batch_slice(const SliceRule& r, const float* __restrict__ t, const pcr_batch& h) {
+    float w = t[15];
+#pragma unroll
+    for (int a = 0; a < 3; a++) w += fminf(t[4 * a + 3] * h.min[a], t[4 * a + 3] * h.max[a]);
+    // a depth at or below 0 has no logarithm: NaN and -infinity clamp to slice 0
+    const float k = __builtin_amdgcn_logf(w * r.inv_near) * r.scale;
+    return (uint32_t)fminf(fmaxf(k, 0.0f), (float)(kSlices - 1));
+}
+
 __device__ __forceinline__ void fill_words(const FillRegion& f, uint64_t t, uint64_t stride) {
     u32x4* p4 = reinterpret_cast<u32x4*>(f.p);
     for (uint64_t i = t; i < f.n / 4; i += stride) p4[i] = u32x4{f.v, f.v, f.v, f.v};
@@ -136,7 +154,7 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(const pcr_batch* __rest
                                                          uint32_t b0, uint32_t b1,
                                                          uint8_t* __restrict__ levels, uint32_t* __restrict__ list,
                                                          FrameState* __restrict__ st, FrameState* __restrict__ st_next,
-                                                         FillRegion fill0, FillRegion fill1) {
+                                                         FillRegion fill0, FillRegion fill1, SliceRule rule_s) {
     constexpr int kWaves = kSelectBlock / 64;
     {
         const uint64_t t = (uint64_t)blockIdx.x * kSelectBlock + threadIdx.x;
@@ -146,15 +164,15 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(const pcr_batch* __rest
         fill_words(fill1, t, stride);
     }
     __shared__ float planes[6][4];   // the view's frustum planes, computed once per workgroup
-    __shared__ uint32_t s_keep[kWaves];
+    __shared__ uint32_t s_keep[kSlices][kWaves];
     __shared__ unsigned long long s_stat[8][kWaves];   // culled, level 0..4, points, bytes
-    __shared__ uint32_t s_base;
+    __shared__ uint32_t s_base[kSlices];
     if (threadIdx.x < 6) frustum_plane(v.transform_frustum, (int)threadIdx.x, planes[threadIdx.x]);
     __syncthreads();
     const uint32_t i = blockIdx.x * kSelectBlock + threadIdx.x;
     const bool in_range = i < nb && i >= b0 && i < b1;   // [b0, b1): the batches of this draw
     int level = kCulled;
-    uint32_t np = 0;
+    uint32_t np = 0, slice = 0;
     if (in_range) {
         const pcr_batch h = b[i];
         bool vis = !culling || planes_visible(planes, h.min, h.max);
@@ -171,12 +189,22 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(const pcr_batch* __rest
                 }
             }
         }
-        if (vis) { level = precision_level(h.min, h.max, v, first); np = h.num_points; }
+        if (vis) {
+            level = precision_level(h.min, h.max, v, first);
+            np = h.num_points;
+            slice = batch_slice(rule_s, v.transform, h);
+        }
     }
     if (i < nb) levels[i] = (uint8_t)level;
     const bool keep = level != kCulled;
-    const unsigned long long m = __ballot(keep);
     const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
+    unsigned long long m = 0;   // the wave's kept batches of this one's slice
+#pragma unroll
+    for (uint32_t k = 0; k < kSlices; k++) {
+        const unsigned long long mk = __ballot(keep && slice == k);
+        if (slice == k) m = mk;
+        if (lane == 0) s_keep[k][wave] = (uint32_t)__popcll(mk);
+    }
     const uint32_t culled = (uint32_t)__popcll(__ballot(in_range && !keep));
     uint32_t cnt[5];
 #pragma unroll
@@ -185,7 +213,6 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(const pcr_batch* __rest
     const unsigned long long bytes =
         wave_sum_u64(keep ? (unsigned long long)np * 4ull * planes_for_level(level) : 0ull);
     if (lane == 0) {
-        s_keep[wave] = (uint32_t)__popcll(m);
         s_stat[0][wave] = culled;
 #pragma unroll
         for (int L = 0; L < 5; L++) s_stat[1 + L][wave] = cnt[L];
@@ -193,10 +220,10 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(const pcr_batch* __rest
         s_stat[7][wave] = bytes;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < kSlices) {
         uint32_t total = 0;
-        for (int w = 0; w < kWaves; w++) total += s_keep[w];
-        s_base = total ? atomicAdd(&st->list_count, total) : 0u;
+        for (int w = 0; w < kWaves; w++) total += s_keep[threadIdx.x][w];
+        s_base[threadIdx.x] = total ? atomicAdd(&st->slice_count[threadIdx.x], total) : 0u;
     } else if (threadIdx.x >= 64 && threadIdx.x < 72) {
         const int k = (int)threadIdx.x - 64;
         unsigned long long sum = 0;
@@ -210,10 +237,31 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(const pcr_batch* __rest
     }
     __syncthreads();
     if (keep) {
-        uint32_t base = s_base;
-        for (uint32_t w = 0; w < wave; w++) base += s_keep[w];
-        list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = i;
+        uint32_t base = s_base[slice];
+        for (uint32_t w = 0; w < wave; w++) base += s_keep[slice][w];
+        list[(uint64_t)slice * nb + base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = i;
     }
+}
+
+// Slices from the nearest to the farthest view depth of the cloud's box, at
+// most a factor of 256 (a box that reaches the eye has no nearest depth), so
+// that each slice spans at most a factor of 2.
+static SliceRule slice_rule(const pcr_cloud* c, const pcr_view& v) {
+    SliceRule r{1.0f, 0.0f};
+    if (c->list_slices != kSlices) return r;
+    double lo = v.transform[15], hi = lo;
+    for (int a = 0; a < 3; a++) {
+        const double x = (double)v.transform[4 * a + 3] * c->aabb_min[a], y = (double)v.transform[4 * a + 3] * c->aabb_max[a];
+        lo += x < y ? x : y;
+        hi += x < y ? y : x;
+    }
+    if (!(hi > 1e-30 && hi < 1e30)) return r;
+    if (!(lo > hi / 256)) lo = hi / 256;
+    const double span = std::log2(hi / lo);
+    if (!(span > 1e-3)) return r;
+    r.inv_near = (float)(1.0 / lo);
+    r.scale = (float)(kSlices / span);
+    return r;
 }
 
 int launch_select(hipStream_t s, const pcr_cloud* c, const pcr_view& v, const pcr_render_params& p,
@@ -226,14 +274,15 @@ int launch_select(hipStream_t s, const pcr_cloud* c, const pcr_view& v, const pc
     if (fg > 512) fg = 512;
     const int grid = (int)(sel > fg ? sel : (fg ? fg : 1));
     const uint32_t b0 = p.batch_begin, b1 = p.batch_end ? p.batch_end : c->num_batches;
+    const SliceRule sr = slice_rule(c, v);
     if (lod)
         k_select<true><<<grid, kSelectBlock, 0, s>>>(c->d_batches, c->num_batches, v, p.frustum_culling, p.lod_rule,
                                                      p.lod_px, first, b0, b1, c->d_levels, c->d_list, st, st_next,
-                                                     fill0, fill1);
+                                                     fill0, fill1, sr);
     else
         k_select<false><<<grid, kSelectBlock, 0, s>>>(c->d_batches, c->num_batches, v, p.frustum_culling,
                                                       p.lod_rule, p.lod_px, first, b0, b1, c->d_levels, c->d_list,
-                                                      st, st_next, fill0, fill1);
+                                                      st, st_next, fill0, fill1, sr);
     PCR_HIP(hipGetLastError());
     return PCR_OK;
 }
@@ -546,6 +595,226 @@ __device__ __forceinline__ RectInfo uniform_rect(const RectInfo& s) {
     return r;
 }
 
+// The order in which a launch's persistent workgroups draw `count` listed
+// batches, as work items of whole batches or of parts of one.
+//
+// The last nsplit batches (one per workgroup) are drawn in parts: workgroups
+// otherwise idle 43 us on average between their last batch and the end of
+// the launch, and the halves shorten the batches taken last (splitting twice
+// as many items costs more in extra flushes than it saves). With fewer
+// batches than half the workgroups every batch is split further, into as
+// many parts as give each workgroup one: a batch is otherwise ten or more
+// rounds of one workgroup while the rest of the chip is idle. First come the
+// first parts of all of them, then the second ones, and so on, so that a
+// pair of queue items never holds two parts of one batch. The raster of 10
+// batches of 10,240 points takes 8.5 us so, and 42 in two parts each; the hqs
+// passes over 350 octree nodes 78 + 116 us, and 184 + 140. From half the
+// workgroups on, two parts are as good as more (1,821 nodes: 228 us, 252 with
+// the old order of the parts).
+//
+// Consecutive items map to list slots spread over the whole list
+// (multiplying by a prime above any count, modulo the count, permutes the
+// slots), so the batches in flight at one time come from distant parts of
+// the Morton order and cover different screen regions: fewer of their
+// atomics meet on the same framebuffer lines.
+//
+// The slices of the list (SliceRule) are drawn one after the other, the
+// nearest first; the spread is within a slice.
+constexpr uint32_t kMaxParts = 16;
+struct WorkItems {
+    uint32_t count, whole, nsplit, nparts, items;
+    // `start` (LDS, kSlices + 1 words) takes the first item of each slice;
+    // every thread of the workgroup constructs it (it ends in a barrier)
+    __device__ __forceinline__ WorkItems(const FrameState* st, uint32_t* start) {
+        if (threadIdx.x == 0) {
+            uint32_t n = 0;
+            for (uint32_t k = 0; k < kSlices; k++) {
+                start[k] = n;
+                n += st->slice_count[k];
+            }
+            start[kSlices] = n;
+        }
+        __syncthreads();
+        count = __builtin_amdgcn_readfirstlane(start[kSlices]);
+        nsplit = min(count, gridDim.x);
+        whole = count - nsplit;
+        nparts = count * 2u <= gridDim.x && count ? min(kMaxParts, gridDim.x / count) : 2u;
+        items = whole + nsplit * nparts;
+    }
+    // place in a list of nb entries a slice, part and number of parts of an item
+    __device__ __forceinline__ uint64_t slot(uint32_t item, const uint32_t* start, uint32_t nb, uint32_t& part,
+                                             uint32_t& parts) const {
+        part = 0;
+        parts = 1;
+        if (item >= whole) {
+            const uint32_t h = item - whole;
+            part = h / nsplit;
+            parts = nparts;
+            item = whole + (h - part * nsplit);
+        }
+        const unsigned long long m = __ballot(item >= start[__lane_id() & (kSlices - 1)]) & ((1ull << kSlices) - 1);
+        const uint32_t k = (uint32_t)__popcll(m) - 1u;   // empty slices start where the next one does
+        const uint32_t s0 = __builtin_amdgcn_readfirstlane(start[k]), n = __builtin_amdgcn_readfirstlane(start[k + 1]) - s0;
+        return (uint64_t)k * nb + (uint32_t)(((uint64_t)(item - s0) * 2654435761ull) % n);
+    }
+};
+// The points of one part of a batch: whole groups of 1024 points, one round of
+// a 256-thread workgroup (counted from the aligned word that the point loops
+// start at), so that no part ends in a round with idle threads. A part past
+// the last group is empty.
+__device__ __forceinline__ void batch_part(pcr_batch& h, uint32_t part, uint32_t nparts) {
+    constexpr uint32_t kRound = 1024;
+    const uint32_t lead = h.first_point & 3u, rounds = (uint32_t)(((uint64_t)h.num_points + lead + kRound - 1) / kRound);
+    const uint64_t k = (uint64_t)((rounds + nparts - 1) / nparts) * kRound;   // words per part
+    const uint64_t w0 = k * part, end = (uint64_t)h.num_points + lead;
+    const uint64_t lo = w0 > lead ? w0 - lead : 0, hi = w0 + k < end ? w0 + k - lead : h.num_points;
+    h.first_point += (uint32_t)(lo < h.num_points ? lo : h.num_points);
+    h.num_points = lo < hi ? (uint32_t)(hi - lo) : 0u;
+}
+
+// A persistent workgroup's next work item. The first is its own block index;
+// the others come from the launch's queue counter. Every workgroup increments
+// the one counter, and the memory performs atomics on one address one after
+// the other, so a workgroup takes two items per atomic and draws them one
+// after the other (with the split parts ordered as in WorkItems, the
+// 1e9-point 100 m flythrough's raster is 4.7% faster than with one item per
+// atomic, and three or four items are no better), and a launch that gives
+// every item to a workgroup of its own takes none. take() is called by every
+// thread of the workgroup; the returned item is workgroup-uniform. `s_item`
+// must not be rewritten before the workgroup's next barrier.
+struct QueueTake {
+    uint32_t next;                 // the next item that is the workgroup's already, or none
+    __device__ __forceinline__ QueueTake() : next(blockIdx.x) {}
+    __device__ __forceinline__ uint32_t take(uint32_t* head, uint32_t& s_item, uint32_t items) {
+        if (next != 0xFFFFFFFFu) {
+            const uint32_t it = next;
+            next = 0xFFFFFFFFu;
+            return it;
+        }
+        if (items <= gridDim.x) return items;
+        if (threadIdx.x == 0) s_item = atomicAdd(head, 2u);
+        __syncthreads();
+        const uint32_t it = gridDim.x + __builtin_amdgcn_readfirstlane(s_item);
+        next = it + 1u;
+        return it;
+    }
+};
+
+// The groups of a batch that its tile may still need, and the words the
+// workgroup decides it with.
+template <int BLOCK>
+struct GroupList {
+    uint32_t open[BLOCK / 64], closed[BLOCK / 64];   // per wave: threads with an open, a closed pixel
+    uint32_t n;                                      // groups in `live`
+    uint32_t skipped;                                // points of the others
+    uint32_t live[BLOCK];
+    int4 part[BLOCK / 16];                           // batch_range: x0, y0, x1, y1 of 16 groups
+    float part_w[BLOCK / 16];                        // and a depth none of their points undercuts
+};
+
+// Loads the framebuffer's keys over a rectangle of n pixels into the tile.
+// The tile then holds what the rectangle has at this moment: a point behind
+// it fails lds_min's first read, and the flush issues an atomic only for the
+// pixels that changed. Returns 0 when no pixel may take a point at depth wlo
+// or beyond (the batch is hidden; rect_open has the reasons), 1 when some may,
+// 2 when also at least a quarter of the threads hold a pixel that may not.
+// Ends in a barrier.
+template <int BLOCK>
+__device__ __forceinline__ int tile_preload(unsigned long long* tile, const unsigned long long* __restrict__ fb, int x0,
+                                            int y0, int tw, int n, uint32_t magic, uint32_t width, uint32_t wb,
+                                            GroupList<BLOCK>& gl) {
+    bool open = false, closed = false;
+    for (int i = threadIdx.x; i < n; i += BLOCK) {
+        const uint32_t uy = __umulhi((uint32_t)i, magic), ux = (uint32_t)i - uy * (uint32_t)tw;
+        const unsigned long long k = fb[(uint32_t)x0 + ux + ((uint32_t)y0 + uy) * width];
+        tile[i] = k;
+        const bool o = (uint32_t)(k >> 32) >= wb;
+        open |= o;
+        closed |= !o;
+    }
+    const unsigned long long mo = __ballot(open), mc = __ballot(closed);
+    if (__lane_id() == 0) {
+        gl.open[threadIdx.x >> 6] = (uint32_t)__popcll(mo);
+        gl.closed[threadIdx.x >> 6] = (uint32_t)__popcll(mc);
+    }
+    if (threadIdx.x == 0) gl.n = gl.skipped = 0;
+    __syncthreads();
+    uint32_t no = 0, nc = 0;
+#pragma unroll
+    for (int w = 0; w < BLOCK / 64; w++) {
+        no += gl.open[w];
+        nc += gl.closed[w];
+    }
+    no = __builtin_amdgcn_readfirstlane(no);
+    nc = __builtin_amdgcn_readfirstlane(nc);
+    return no == 0 ? 0 : (nc * 4u >= (uint32_t)min(n, BLOCK) ? 2 : 1);
+}
+
+// tile_loop() for an interior batch at the 10-bit level whose tile was
+// preloaded, without the groups of 64 points that lie behind the tile's
+// depths everywhere (VALU-bound: a point costs some 45 instructions, a
+// group's test about four points' worth): one thread tests one group's rectangle against the tile
+// (group_rect bounds where its points land and how near they are; the
+// reasoning is rect_open's), then 16 lanes draw each remaining group.
+// A group over more than kGroupTestPix pixels is drawn untested: its test
+// would cost more than its points.
+constexpr int kGroupTestPix = 64;
+template <int BLOCK, bool NT>
+__device__ __forceinline__ void tile_groups(const Decode& d, const uint32_t* __restrict__ lo,
+                                            const uint2* __restrict__ box, const pcr_batch& h, const pcr_view& v,
+                                            const Proj& pj, GroupSlack slack, unsigned long long* __restrict__ fb,
+                                            unsigned long long* tile, int x0, int y0, int tw, int th, uint32_t* natom,
+                                            GroupList<BLOCK>& gl) {
+    const uint32_t first = h.first_point, np = h.num_points;
+    const uint32_t lead = first & 3u, ng = groups_of(first, np), nq = (np + lead + 3u) >> 2;
+    const u32x4* lo4 = reinterpret_cast<const u32x4*>(lo + (first - lead));
+    for (uint32_t g0 = 0; g0 < ng; g0 += BLOCK) {
+        if (g0) {   // the list of the last BLOCK groups has been drawn
+            __syncthreads();
+            if (threadIdx.x == 0) gl.n = 0;
+            __syncthreads();
+        }
+        const uint32_t g = g0 + threadIdx.x;
+        bool live = g < ng;
+        if (live) {
+            const GroupRect r = group_rect(box[g], 2, d, v.transform, v.width, v.height, slack.px, slack.w);
+            const int rx0 = max(r.x0 - x0, 0), ry0 = max(r.y0 - y0, 0), rx1 = min(r.x1 - x0, tw - 1),
+                      ry1 = min(r.y1 - y0, th - 1);
+            const int rw = rx1 - rx0 + 1, rh = ry1 - ry0 + 1;
+            if (!r.wild && rw > 0 && rh > 0 && rw <= kGroupTestPix && rh <= kGroupTestPix && rw * rh <= kGroupTestPix) {
+                const uint32_t wb = r.w > 0.0f ? __float_as_uint(r.w) : 0u;
+                const uint32_t* t32 = reinterpret_cast<const uint32_t*>(tile) + 1;   // the depths
+                live = false;
+                for (int y = ry0; y <= ry1 && !live; y++)
+                    for (int x = rx0; x <= rx1 && !live; x++) live = t32[2 * (y * tw + x)] >= wb;
+            }
+            if (!live) {
+                const uint32_t end = min((g + 1) * kGroupPoints, np + lead), beg = max(g * kGroupPoints, lead);
+                lds_add32(&gl.skipped, end - beg);
+            }
+        }
+        const unsigned long long m = __ballot(live);
+        uint32_t base = 0;
+        if (__lane_id() == 0 && m)
+            base = __hip_atomic_fetch_add((lds_u32*)&gl.n, (uint32_t)__popcll(m), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_WORKGROUP);
+        base = __builtin_amdgcn_readfirstlane(base);
+        if (live) gl.live[base + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull))] = g;
+        __syncthreads();
+        const uint32_t n = __builtin_amdgcn_readfirstlane(gl.n);
+        for (uint32_t j = threadIdx.x >> 4; j < n; j += BLOCK / 16) {
+            const uint32_t q = gl.live[j] * (kGroupPoints / 4) + (threadIdx.x & 15u);
+            if (q >= nq) continue;
+            const u32x4 a = ld_plane<NT>(lo4 + q);
+            const uint32_t base = q * 4u - lead;
+            tile_point<2, true, true>(d, a.x, 0u, 0u, base + 0, np, first, pj, fb, tile, x0, y0, tw, th, natom);
+            tile_point<2, true, true>(d, a.y, 0u, 0u, base + 1, np, first, pj, fb, tile, x0, y0, tw, th, natom);
+            tile_point<2, true, true>(d, a.z, 0u, 0u, base + 2, np, first, pj, fb, tile, x0, y0, tw, th, natom);
+            tile_point<2, true, true>(d, a.w, 0u, 0u, base + 3, np, first, pj, fb, tile, x0, y0, tw, th, natom);
+        }
+    }
+}
+
 // One batch of the tiled raster; `bi` and `level` are workgroup-uniform.
 // Returns the points skipped by the occlusion test (0 if the batch drew).
 // PRE: the batch's screen rectangle for the view comes in `pre` (the
@@ -559,10 +828,9 @@ __device__ __forceinline__ uint32_t tiled_batch(uint32_t bi, int level, const pc
                                                 uint32_t* natom, bool occl, uint32_t part = 0, uint32_t nparts = 1,
                                                 const RectInfo* pre = nullptr) {
     pcr_batch h = b[bi];
-    if (nparts > 1) {   // points [part * k, (part + 1) * k) of the batch, k = ceil(n / nparts)
-        const uint32_t k = (h.num_points + nparts - 1) / nparts, off = min(part * k, h.num_points);
-        h.first_point += off;
-        h.num_points = min(k, h.num_points - off);
+    if (nparts > 1) {
+        batch_part(h, part, nparts);
+        if (h.num_points == 0) return 0;
     }
     int x0 = 0, y0 = 0, x1 = -1, y1 = -1;
     bool interior, use;
@@ -604,81 +872,211 @@ __device__ __forceinline__ uint32_t tiled_batch(uint32_t bi, int level, const pc
     return 0;
 }
 
-// A persistent workgroup's next queue item. Every workgroup increments the
-// one queue counter, and the memory performs atomics on one address one after
-// the other, so a workgroup takes two items per atomic and draws them one
-// after the other (with the split halves ordered as in k_raster_tiled, the
-// 1e9-point 100 m flythrough's raster is 4.7% faster than with one item per
-// atomic, and three or four items are no better). take() is called by every
-// thread of the workgroup; the returned item is workgroup-uniform. `s_item`
-// must not be rewritten before the workgroup's next barrier.
-struct QueueTake {
-    uint32_t next = 0xFFFFFFFFu;   // the second item of the last pair, not yet drawn
-    __device__ __forceinline__ uint32_t take(uint32_t* head, uint32_t& s_item) {
-        if (next != 0xFFFFFFFFu) {
-            const uint32_t it = next;
-            next = 0xFFFFFFFFu;
-            return it;
+// The rectangles of a batch's parts of 16 groups, for up to BLOCK groups from
+// g0 on, into gl.part: one thread bounds one group, and the 16 lanes of a part
+// join theirs. A part outside the image has an empty rectangle; one without a
+// bound has a rectangle that fits no tile. Ends in a barrier.
+template <int BLOCK>
+__device__ __forceinline__ void batch_parts(const uint2* __restrict__ box, uint32_t g0, uint32_t ng, int level,
+                                            const Decode& d, const pcr_view& v, GroupSlack slack, GroupList<BLOCK>& gl) {
+    constexpr int kOut = 1 << 20;   // beyond any pixel
+    int x0 = kOut, y0 = kOut, x1 = -1, y1 = -1;
+    float w = 3e38f;
+    if (g0 + threadIdx.x < ng) {
+        const GroupRect r = group_rect(box[g0 + threadIdx.x], level, d, v.transform, v.width, v.height, slack.px, slack.w);
+        if (r.wild) {
+            x0 = y0 = 0;
+            x1 = y1 = kOut;
+            w = 0.0f;
+        } else if (r.x1 >= r.x0 && r.y1 >= r.y0) {
+            x0 = r.x0; y0 = r.y0; x1 = r.x1; y1 = r.y1;
+            w = r.w;
         }
-        if (threadIdx.x == 0) s_item = atomicAdd(head, 2u);
-        __syncthreads();
-        const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
-        next = it + 1u;
-        return it;
     }
-};
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1) {
+        x0 = min(x0, __shfl_xor(x0, m));
+        y0 = min(y0, __shfl_xor(y0, m));
+        x1 = max(x1, __shfl_xor(x1, m));
+        y1 = max(y1, __shfl_xor(y1, m));
+        w = fminf(w, __shfl_xor(w, m));
+    }
+    __syncthreads();   // the last parts have been drawn
+    if ((threadIdx.x & 15u) == 0) {
+        gl.part[threadIdx.x >> 4] = make_int4(x0, y0, x1, y1);
+        gl.part_w[threadIdx.x >> 4] = fmaxf(w, 0.0f);
+    }
+    __syncthreads();
+}
+
+// One batch of the tiled raster for a cloud with group bounds; `bi` and
+// `level` are workgroup-uniform. Returns the points skipped by the occlusion
+// tests. A batch whose rectangle fits the tile is drawn in one piece. A larger
+// one (a near batch, whose points are spread widely) is drawn in runs of parts
+// of 16 groups: its points are in Morton order, so a part covers about its
+// share of the rectangle, and a run whose rectangle fits the tile is merged
+// there and flushed in rows, whose pixels share requests. Drawn point by point
+// such batches are bound by the requests that the memory takes (25 G/s over the
+// whole chip, one per 64-byte line of an atomic instruction). A single part
+// that does not fit is drawn point by point: with fewer points than half its
+// pixels, few share a line. Parts outside the image are left out.
+//
+// Measured, with the near-first slices: the 1e9-point city from 100 m
+// (1920x1080, 19,494 batches drawn) 419 -> 333 us a frame, with 2.9 -> 0.8 M
+// atomic requests and 57% of the points left out (19% before); from above
+// (96,853 batches) 1,284 -> 1,135 us; 1,821 nodes of an octree 261 -> 236 us.
+// The slices and the group test alone gave 410, 1,020 and 262: the registers
+// of the parts cost the overview a fifth wave per SIMD's worth of latency. A
+// kernel of its own for the large batches, before this one, was slower (443
+// us): its waits for memory no longer overlap the other batches' arithmetic.
+template <int BLOCK, int TILE_PIX>
+__device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const pcr_batch* __restrict__ b,
+                                                  const uint32_t* __restrict__ lo, const uint32_t* __restrict__ med,
+                                                  const uint32_t* __restrict__ hi, const pcr_view& v,
+                                                  unsigned long long* __restrict__ fb, unsigned long long* tile,
+                                                  uint32_t* natom, bool occl, uint32_t part, uint32_t nparts,
+                                                  const uint2* __restrict__ box, GroupList<BLOCK>& gl) {
+    pcr_batch h = b[bi];
+    if (nparts > 1) {
+        const uint32_t f = h.first_point & ~3u;
+        batch_part(h, part, nparts);
+        if (h.num_points == 0) return 0;
+        box += ((h.first_point & ~3u) - f) / kGroupPoints;   // parts are whole groups
+    }
+    int x0 = 0, y0 = 0, x1 = -1, y1 = -1;
+    bool interior;
+    float wlo, wnear;
+    bool use = screen_rect(v.transform, h.min, h.max, v.width, v.height, x0, y0, x1, y1, &interior, &wlo, &wnear);
+    int tw = x1 - x0 + 1, th = y1 - y0 + 1;
+    const auto fits = [](int w, int hh) { return w >= 2 && w <= TILE_PIX && hh <= TILE_PIX && w * hh <= TILE_PIX; };
+    const bool parted = use && !fits(tw, th) && wnear > 0.0f;
+    const uint32_t first = h.first_point, np = h.num_points, lead = first & 3u, ng = groups_of(first, np);
+    uint32_t skipped = 0, g = 0;   // g: the first group not yet drawn
+    for (;;) {
+        bool tests = occl && wlo > 0.0f;
+        if (parted) {
+            const uint32_t p0 = (g & (BLOCK - 1u)) >> 4;
+            if (p0 == 0)
+                batch_parts<BLOCK>(box, g, ng, level, make_decode(level, h.min, h.max), v,
+                                   group_slack(v.transform, h.min, h.max, v.width, v.height, wnear), gl);
+            const uint32_t left = min((ng - g + 15u) >> 4, BLOCK / 16u - p0);
+            int r[4] = {gl.part[p0].x, gl.part[p0].y, gl.part[p0].z, gl.part[p0].w};
+            float w = gl.part_w[p0];
+            uint32_t n = 1;
+            for (; n < left; n++) {   // join the next part while the rectangle fits
+                const int4 q = gl.part[p0 + n];
+                const int a0 = min(r[0], q.x), a1 = min(r[1], q.y), a2 = max(r[2], q.z), a3 = max(r[3], q.w);
+                if (a2 >= 0 && !fits(max(a2 - a0 + 1, 2), a3 - a1 + 1)) break;
+                r[0] = a0; r[1] = a1; r[2] = a2; r[3] = a3;
+                w = fminf(w, gl.part_w[p0 + n]);
+            }
+            n = __builtin_amdgcn_readfirstlane(n);
+            x0 = __builtin_amdgcn_readfirstlane(r[0]);
+            y0 = __builtin_amdgcn_readfirstlane(r[1]);
+            tw = __builtin_amdgcn_readfirstlane(r[2]) - x0 + 1;
+            th = __builtin_amdgcn_readfirstlane(r[3]) - y0 + 1;
+            wlo = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(w)));
+            const uint32_t w0 = g * kGroupPoints, w1 = (g + n * 16u) * kGroupPoints;
+            const uint32_t o0 = w0 > lead ? w0 - lead : 0u, o1 = min(w1 - lead, np);
+            h.first_point = first + o0;
+            h.num_points = o1 - o0;
+            g += n * 16u;
+            tests = occl;
+            use = fits(tw, th);
+            if (tw <= 0) {   // outside the image
+                if (g >= ng) break;
+                continue;
+            }
+        } else {
+            use = use && fits(tw, th);
+        }
+        const int n = tw * th;
+        const uint32_t magic = use ? row_magic(tw) : 0u;
+        int seen = 1;
+        if (use) {
+            if (tests) {
+                seen = tile_preload<BLOCK>(tile, fb, x0, y0, tw, n, magic, (uint32_t)v.width, __float_as_uint(wlo), gl);
+            } else {
+                for (int i = threadIdx.x; i < n; i += BLOCK) tile[i] = PCR_FB_CLEAR;
+                __syncthreads();
+            }
+        }
+        if (seen == 0) {
+            skipped += h.num_points;
+        } else {
+            const Decode d = make_decode(level, h.min, h.max);
+            const Proj pj = make_proj(v.transform, v.width, v.height);
+            if (use) {
+                if (seen == 2 && level >= 2 && interior) {
+                    tile_groups<BLOCK, true>(d, lo, parted ? box + (h.first_point - (h.first_point & 3u) - (first - lead)) / kGroupPoints : box,
+                                             h, v, pj, group_slack(v.transform, h.min, h.max, v.width, v.height, wnear),
+                                             fb, tile, x0, y0, tw, th, natom, gl);
+                } else {
+                    tile_dispatch<BLOCK, true, true>(level, d, lo, med, hi, h, pj, fb, tile, x0, y0, tw, th, natom,
+                                                     interior);
+                }
+                __syncthreads();
+                if (tests) skipped += gl.skipped;
+                tile_flush<BLOCK>(tile, fb, x0, y0, tw, n, magic, (uint32_t)v.width, natom);
+            } else {
+                tile_dispatch<BLOCK, false, true>(level, d, lo, med, hi, h, pj, fb, nullptr, 0, 0, 0, 0, natom);
+            }
+        }
+        if (!parted || g >= ng) break;
+        __syncthreads();   // the tile is reused by the next run
+    }
+    return skipped;
+}
 
 // Persistent workgroups take drawn batches from the select stage's compacted
 // list through an atomic queue, so no workgroup is launched for a culled
 // batch. The loop ends when the queue passes list_count, which every
 // workgroup reaches.
-template <int BLOCK, int TILE_PIX>
-__global__ __launch_bounds__(BLOCK) void k_raster_tiled(const pcr_batch* __restrict__ b,
+// GROUPS: the cloud has group bounds. Six waves per SIMD: with eight the
+// batch state spills inside the loops (361 us for the frame above, 340 with
+// seven, 333 with six).
+template <int BLOCK, int TILE_PIX, bool GROUPS>
+__global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_raster_tiled(const pcr_batch* __restrict__ b,
                                                         const uint8_t* __restrict__ levels,
                                                         const uint32_t* __restrict__ list,
                                                         FrameState* __restrict__ st,
                                                         const uint32_t* __restrict__ lo,
                                                         const uint32_t* __restrict__ med,
                                                         const uint32_t* __restrict__ hi, pcr_view v,
-                                                        unsigned long long* __restrict__ fb, int occl) {
+                                                        unsigned long long* __restrict__ fb, int occl,
+                                                        uint32_t nb, const uint2* __restrict__ gbox,
+                                                        const uint32_t* __restrict__ gbase) {
     __shared__ unsigned long long tile[TILE_PIX];
     __shared__ uint32_t s_item, s_occ_batches, s_natom;   // s_natom: framebuffer atomics issued
     __shared__ unsigned long long s_occ_points, s_occ_bytes;   // what the occlusion test skipped
-    const uint32_t count = st->list_count;
-    const uint32_t nsplit = min(count, gridDim.x), whole = count - nsplit;
+    __shared__ uint32_t s_start[kSlices + 1];
+    __shared__ GroupList<BLOCK> groups;
+    const WorkItems work(st, s_start);
     if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; s_natom = 0; }
+    __syncthreads();
     QueueTake q;
     for (;;) {
-        uint32_t item = q.take(&st->queue_head, s_item);
-        if (item >= count + nsplit) break;
-        // The last nsplit batches (one per workgroup) are drawn as two halves
-        // each: workgroups otherwise idle 43 us on average between their
-        // last batch and the end of the launch, and the halves shorten the
-        // batches taken last (splitting twice as many items costs more in
-        // extra flushes than it saves). The first halves of all of them come
-        // first, then the second halves, so that a pair of queue items never
-        // holds both halves of one batch.
-        uint32_t part = 0, nparts = 1;
-        if (item >= whole) {
-            const uint32_t h = item - whole;
-            part = h >= nsplit ? 1u : 0u;
-            nparts = 2;
-            item = whole + (part ? h - nsplit : h);
-        }
-        // Consecutive queue items map to list slots spread over the whole list
-        // (multiplying by a prime above any count, modulo the count, permutes
-        // the slots), so the batches in flight at one time come from distant
-        // parts of the Morton order and cover different screen regions: fewer
-        // of their atomics meet on the same framebuffer lines.
-        const uint32_t slot = (uint32_t)(((uint64_t)item * 2654435761ull) % count);
+        const uint32_t item = q.take(&st->queue_head, s_item, work.items);
+        if (item >= work.items) break;
+        uint32_t part, nparts;
+        const uint64_t slot = work.slot(item, s_start, nb, part, nparts);
         const uint32_t bi = __builtin_amdgcn_readfirstlane(list[slot]);
         const int level = __builtin_amdgcn_readfirstlane(levels[bi]);
-        const uint32_t skipped = tiled_batch<BLOCK, TILE_PIX, true>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom,
-                                                                    occl != 0, part, nparts);
+        uint32_t skipped;
+        if constexpr (GROUPS)
+            skipped = grouped_batch<BLOCK, TILE_PIX>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0, part,
+                                                     nparts, gbox + gbase[bi], groups);
+        else
+            skipped = tiled_batch<BLOCK, TILE_PIX, true>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0,
+                                                         part, nparts);
         if (threadIdx.x == 0 && skipped) {
             s_occ_points += skipped;
             s_occ_bytes += 4ull * planes_for_level(level) * skipped;
-            s_occ_batches += part == 0;   // a batch drawn as two halves counts once
+            if (part == 0) {   // a batch drawn in parts counts once, by its first
+                pcr_batch h = b[bi];
+                if (nparts > 1) batch_part(h, 0, nparts);
+                s_occ_batches += skipped == h.num_points;
+            }
         }
         __syncthreads();   // s_item and the tile are reused by the next item
     }
@@ -691,21 +1089,29 @@ __global__ __launch_bounds__(BLOCK) void k_raster_tiled(const pcr_batch* __restr
     }
 }
 
-template <int BLOCK, int TILE_PIX>
-static void tiled_t(hipStream_t s, const pcr_cloud* c, const pcr_view& v, FrameState* st, unsigned long long* fb,
+template <int BLOCK, int TILE_PIX, bool GROUPS>
+static void tiled_grid(hipStream_t s, const pcr_cloud* c, const pcr_view& v, FrameState* st, unsigned long long* fb,
                     bool occl) {
     static const int occ = [] {
         int o = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, k_raster_tiled<BLOCK, TILE_PIX>, BLOCK, 0) != hipSuccess) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, k_raster_tiled<BLOCK, TILE_PIX, GROUPS>, BLOCK, 0) != hipSuccess) {
             (void)hipGetLastError();
             o = 0;
         }
         return o > 0 ? o : 4;
     }();
     uint64_t grid = (uint64_t)c->ctx->cu_count * (uint64_t)occ;
-    if (grid > c->num_batches) grid = c->num_batches;
-    k_raster_tiled<BLOCK, TILE_PIX><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->d_levels, c->d_list, st, c->d_lo,
-                                                               c->d_med, c->d_hi, v, fb, occl ? 1 : 0);
+    if (grid > (uint64_t)c->num_batches * kMaxParts) grid = (uint64_t)c->num_batches * kMaxParts;
+    k_raster_tiled<BLOCK, TILE_PIX, GROUPS><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->d_levels, c->d_list, st, c->d_lo,
+                                                               c->d_med, c->d_hi, v, fb, occl ? 1 : 0,
+                                                               c->num_batches, c->d_gbox, c->d_gbase);
+}
+
+template <int BLOCK, int TILE_PIX>
+static void tiled_t(hipStream_t s, const pcr_cloud* c, const pcr_view& v, FrameState* st, unsigned long long* fb,
+                    bool occl) {
+    if (c->d_gbox) tiled_grid<BLOCK, TILE_PIX, true>(s, c, v, st, fb, occl);
+    else tiled_grid<BLOCK, TILE_PIX, false>(s, c, v, st, fb, occl);
 }
 
 int launch_raster_tiled(hipStream_t s, const pcr_cloud* c, const pcr_view& v, int tile_px, int block,
@@ -798,11 +1204,7 @@ __device__ __forceinline__ bool raster_pair_batch(uint32_t bi, int level, const 
                                                   uint32_t* natom, bool occl, uint32_t part, uint32_t nparts,
                                                   const RectInfo& ra, const RectInfo& rb) {
     pcr_batch h = b[bi];
-    if (nparts > 1) {   // as in tiled_batch
-        const uint32_t k = (h.num_points + nparts - 1) / nparts, off = min(part * k, h.num_points);
-        h.first_point += off;
-        h.num_points = min(k, h.num_points - off);
-    }
+    if (nparts > 1) batch_part(h, part, nparts);
     const int ax0 = ra.x0, ay0 = ra.y0, bx0 = rb.x0, by0 = rb.y0;
     const bool aon = ra.on != 0, bon = rb.on != 0, ai = ra.interior != 0, bi_ = rb.interior != 0;
     const float awlo = ra.wlo, bwlo = rb.wlo;
@@ -1195,10 +1597,9 @@ __device__ __forceinline__ uint32_t hqs_tiled_batch(uint32_t bi, int level, cons
                                                 uint32_t nparts = 1) {
     const pcr_batch h = b[bi];
     pcr_batch hp = h;   // the points this item draws; the tile and band choices follow the whole batch
-    if (nparts > 1) {   // points [part * k, (part + 1) * k), k = ceil(n / nparts)
-        const uint32_t k = (h.num_points + nparts - 1) / nparts, off = min(part * k, h.num_points);
-        hp.first_point += off;
-        hp.num_points = min(k, h.num_points - off);
+    if (nparts > 1) {
+        batch_part(hp, part, nparts);
+        if (hp.num_points == 0) return 0;
     }
     const Decode d = make_decode(level, h.min, h.max);
     const Proj pj = make_proj(v.transform, v.width, v.height);
@@ -1323,11 +1724,7 @@ __device__ __forceinline__ bool hqs1_pair_batch(uint32_t bi, int level, const pc
                                                 uint32_t* tdepth_b, bool occl, uint32_t part, uint32_t nparts) {
     const pcr_batch h = b[bi];
     pcr_batch hp = h;   // as in hqs_tiled_batch: the points this item draws
-    if (nparts > 1) {
-        const uint32_t k = (h.num_points + nparts - 1) / nparts, off = min(part * k, h.num_points);
-        hp.first_point += off;
-        hp.num_points = min(k, h.num_points - off);
-    }
+    if (nparts > 1) batch_part(hp, part, nparts);
     int ax0 = 0, ay0 = 0, ax1 = -1, ay1 = -1, bx0 = 0, by0 = 0, bx1 = -1, by1 = -1;
     bool ai, bi_;
     float awlo, bwlo;
@@ -1444,11 +1841,7 @@ __device__ __forceinline__ bool hqs2_pair_batch(uint32_t bi, int level, const pc
                                                 uint32_t nparts) {
     const pcr_batch h = b[bi];
     pcr_batch hp = h;   // as in hqs_tiled_batch: the points this item draws
-    if (nparts > 1) {
-        const uint32_t k = (h.num_points + nparts - 1) / nparts, off = min(part * k, h.num_points);
-        hp.first_point += off;
-        hp.num_points = min(k, h.num_points - off);
-    }
+    if (nparts > 1) batch_part(hp, part, nparts);
     int ax0 = 0, ay0 = 0, ax1 = -1, ay1 = -1, bx0 = 0, by0 = 0, bx1 = -1, by1 = -1;
     bool ai, bi_;
     float awlo, bwlo;
@@ -1502,29 +1895,22 @@ void k_hqs_tiled(const pcr_batch* __restrict__ b,
                  const uint32_t* __restrict__ hi,
                  const uint32_t* __restrict__ rgba, pcr_view v,
                  uint32_t* __restrict__ depth,
-                 uint32_t* __restrict__ acc, int occl) {
+                 uint32_t* __restrict__ acc, int occl, uint32_t nb) {
     __shared__ HqsTile<PASS, TILE_PIX> tile;
     __shared__ uint32_t s_item;
     uint32_t* head = PASS == 0 ? &st->queue_head : &st->queue_head2;
-    const uint32_t count = st->list_count;
-    const uint32_t nsplit = min(count, gridDim.x), whole = count - nsplit;
+    __shared__ uint32_t s_start[kSlices + 1];
+    const WorkItems work(st, s_start);
     __shared__ uint32_t s_occ_batches;
     __shared__ unsigned long long s_occ_points, s_occ_bytes;   // what the occlusion test skipped
     if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; }
+    __syncthreads();
     QueueTake q;
     for (;;) {
-        uint32_t item = q.take(head, s_item);
-        if (item >= count + nsplit) break;
-        // as in k_raster_tiled, the last nsplit batches are drawn as two halves,
-        // all first halves before the second ones
-        uint32_t part = 0, nparts = 1;
-        if (item >= whole) {
-            const uint32_t h = item - whole;
-            part = h >= nsplit ? 1u : 0u;
-            nparts = 2;
-            item = whole + (part ? h - nsplit : h);
-        }
-        const uint32_t slot = (uint32_t)(((uint64_t)item * 2654435761ull) % count);
+        const uint32_t item = q.take(head, s_item, work.items);
+        if (item >= work.items) break;
+        uint32_t part, nparts;
+        const uint64_t slot = work.slot(item, s_start, nb, part, nparts);
         const uint32_t bi = __builtin_amdgcn_readfirstlane(list[slot]);
         const int level = __builtin_amdgcn_readfirstlane(levels[bi]);
         const uint32_t skipped = hqs_tiled_batch<BLOCK, TILE_PIX, PASS, true>(bi, level, b, lo, med, hi, rgba, v,
@@ -1557,10 +1943,10 @@ static void hqs_tiled_t(hipStream_t s, const pcr_cloud* c, const pcr_view& v, Fr
         return o > 0 ? o : 4;
     }();
     uint64_t grid = (uint64_t)c->ctx->cu_count * (uint64_t)occ;
-    if (grid > c->num_batches) grid = c->num_batches;
+    if (grid > (uint64_t)c->num_batches * kMaxParts) grid = (uint64_t)c->num_batches * kMaxParts;
     k_hqs_tiled<BLOCK, TILE_PIX, PASS><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->d_levels, c->d_list, st, c->d_lo,
                                                                    c->d_med, c->d_hi, c->d_rgba, v, fb->d_depth,
-                                                                   fb->d_acc, occl ? 1 : 0);
+                                                                   fb->d_acc, occl ? 1 : 0, c->num_batches);
 }
 
 template <int BLOCK, int TILE_PIX>

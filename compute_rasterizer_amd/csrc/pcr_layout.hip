@@ -242,6 +242,8 @@ void cloud_free(pcr_cloud* c) {
     if (!c) return;
     (void)hipFree(c->d_batches); (void)hipFree(c->d_lo); (void)hipFree(c->d_med); (void)hipFree(c->d_hi);
     (void)hipFree(c->d_rgba); (void)hipFree(c->d_points16); (void)hipFree(c->d_levels); (void)hipFree(c->d_list);
+    (void)hipFree(c->d_gbox);   // with the group bases behind the boxes
+    c->d_gbox = nullptr; c->d_gbase = nullptr;
     c->d_batches = nullptr; c->d_lo = c->d_med = c->d_hi = c->d_rgba = nullptr;
     c->d_points16 = nullptr; c->d_levels = nullptr; c->d_list = nullptr;
 }
@@ -257,7 +259,7 @@ int cloud_alloc_batched(pcr_ctx* ctx, uint32_t nb, uint64_t npoints, pcr_cloud* 
     if (hipMalloc(&c->d_batches, nbb * sizeof(pcr_batch)) != hipSuccess ||
         hipMalloc(&c->d_lo, pb) != hipSuccess || hipMalloc(&c->d_med, pb) != hipSuccess ||
         hipMalloc(&c->d_hi, pb) != hipSuccess || hipMalloc(&c->d_rgba, pb) != hipSuccess ||
-        hipMalloc(&c->d_levels, nbb) != hipSuccess || hipMalloc(&c->d_list, nbb * 4) != hipSuccess) {
+        hipMalloc(&c->d_levels, nbb) != hipSuccess || hipMalloc(&c->d_list, nbb * 4 * kSlices) != hipSuccess) {
         (void)hipGetLastError();
         cloud_free(c);
         set_error("device allocation of %llu points / %u batches failed", (unsigned long long)npoints, nb);
@@ -271,7 +273,75 @@ int cloud_alloc_batched(pcr_ctx* ctx, uint32_t nb, uint64_t npoints, pcr_cloud* 
         PCR_HIP(hipMemsetAsync(c->d_hi + npoints, 0, pad * 4, ctx->stream));
         PCR_HIP(hipMemsetAsync(c->d_rgba + npoints, 0, pad * 4, ctx->stream));
     }
-    c->device_bytes = nbb * (sizeof(pcr_batch) + 5) + 4 * pb;
+    c->list_slices = kSlices;
+    c->device_bytes = nbb * (sizeof(pcr_batch) + 1 + 4 * kSlices) + 4 * pb;
+    return PCR_OK;
+}
+
+// Coarse-plane bounds of every group of kGroupPoints points: a 16-lane row of
+// a wave holds one group, a quad of words per lane. blockIdx.x is the batch;
+// the groups of long batches are spread over blockIdx.y. Packed as the plane's
+// words are: min in x, max in y. Bound by the one read of the coarse plane.
+__global__ __launch_bounds__(256) void k_group_box(const pcr_batch* __restrict__ b, const uint32_t* __restrict__ gbase,
+                                                   const uint32_t* __restrict__ lo, uint2* __restrict__ box) {
+    const uint32_t first = b[blockIdx.x].first_point, np = b[blockIdx.x].num_points;
+    const uint32_t lead = first & 3u, ng = groups_of(first, np), nq = (uint32_t)(((uint64_t)np + lead + 3u) >> 2);
+    const u32x4* lo4 = reinterpret_cast<const u32x4*>(lo + (first - lead));
+    for (uint64_t g = blockIdx.y * 16u + (threadIdx.x >> 4); g < ng; g += 16u * gridDim.y) {
+        const uint64_t q = g * (kGroupPoints / 4) + (threadIdx.x & 15u);
+        uint32_t mn[3] = {1023u, 1023u, 1023u}, mx[3] = {0u, 0u, 0u};
+        if (q < nq) {
+            const u32x4 w = lo4[q];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if ((uint32_t)q * 4u + (uint32_t)j - lead < np)
+#pragma unroll
+                    for (int a = 0; a < 3; a++) {
+                        const uint32_t v = (w[j] >> (10 * a)) & 1023u;
+                        mn[a] = min(mn[a], v);
+                        mx[a] = max(mx[a], v);
+                    }
+        }
+#pragma unroll
+        for (int m = 1; m < 16; m <<= 1)
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                mn[a] = min(mn[a], (uint32_t)__shfl_xor((int)mn[a], m));
+                mx[a] = max(mx[a], (uint32_t)__shfl_xor((int)mx[a], m));
+            }
+        if ((threadIdx.x & 15u) == 0)
+            box[gbase[blockIdx.x] + g] =
+                make_uint2(mn[0] | (mn[1] << 10) | (mn[2] << 20), mx[0] | (mx[1] << 10) | (mx[2] << 20));
+    }
+}
+
+int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
+    const uint32_t nb = c->num_batches;
+    if (nb == 0) return PCR_OK;
+    std::vector<uint32_t> base(nb);
+    uint64_t total = 0;
+    uint32_t longest = 0;
+    for (uint32_t i = 0; i < nb; i++) {
+        base[i] = (uint32_t)total;
+        const uint32_t ng = groups_of(c->h_batches[i].first_point, c->h_batches[i].num_points);
+        total += ng;
+        longest = ng > longest ? ng : longest;
+    }
+    if (total == 0 || total >= (1ull << 32)) return PCR_OK;
+    uint2* box = nullptr;
+    if (hipMalloc(&box, total * sizeof(uint2) + nb * sizeof(uint32_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        return PCR_OK;
+    }
+    c->d_gbox = box;
+    c->d_gbase = reinterpret_cast<uint32_t*>(box + total);
+    hipStream_t s = ctx->stream;
+    const uint32_t rows = (longest + 255) / 256 < 256 ? (longest + 255) / 256 : 256;   // 256 groups or more a workgroup
+    PCR_HIP(hipMemcpyAsync(c->d_gbase, base.data(), nb * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+    k_group_box<<<dim3(nb, rows), 256, 0, s>>>(c->d_batches, c->d_gbase, c->d_lo, c->d_gbox);
+    PCR_HIP(hipGetLastError());
+    PCR_HIP(hipStreamSynchronize(s));
+    c->device_bytes += total * sizeof(uint2) + nb * sizeof(uint32_t);
     return PCR_OK;
 }
 
@@ -360,6 +430,8 @@ int build_cloud_device(pcr_ctx* ctx, const float* xyz, const uint32_t* rgba, uin
     if (d_perm) PCR_HIP(hipFree(d_perm));
     c->h_batches.resize(nb);
     PCR_HIP(hipMemcpy(c->h_batches.data(), c->d_batches, sizeof(pcr_batch) * nb, hipMemcpyDeviceToHost));
+    rc = cloud_build_groups(ctx, c);
+    if (rc != PCR_OK) { cloud_free(c); delete c; return rc; }
     *out = c;
     return PCR_OK;
 }

@@ -339,6 +339,8 @@ int build_octree_host(pcr_ctx* ctx, const float* xyz, const uint32_t* rgba, uint
     PCR_HIP(hipMemcpy(c->d_rgba, L.col.data(), np * 4, hipMemcpyHostToDevice));
     PCR_HIP(hipStreamSynchronize(ctx->stream));
     c->h_batches = L.hdr;
+    rc = cloud_build_groups(ctx, c);
+    if (rc) { cloud_free(c); delete c; return rc; }
     *out = c;
     return PCR_OK;
 }

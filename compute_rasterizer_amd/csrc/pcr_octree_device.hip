@@ -627,6 +627,8 @@ int build_octree_device(pcr_ctx* ctx, const float* xyz, const uint32_t* rgba, ui
     PCR_HIP(hipGetLastError());
     PCR_HIP(hipStreamSynchronize(s));
     c->h_batches = std::move(hdr);
+    rc = cloud_build_groups(ctx, c);
+    if (rc) { cloud_free(c); delete c; return rc; }
     *out = c;
     return PCR_OK;
 }

@@ -165,9 +165,10 @@ typedef struct pcr_stats {
                                       because every pixel of the batch's screen
                                       rectangle already held a nearer point (hqs:
                                       both passes, a batch per pass)            */
-    uint64_t points_occluded;      /* the points of those batches                 */
+    uint64_t points_occluded;      /* the points of those batches, and of the 64-point
+                                      groups left out of others for the same reason */
     uint64_t bytes_occluded;       /* the plane bytes (hqs pass 2: and colour
-                                      bytes) those batches did not read; the
+                                      bytes) those points did not take; the
                                       raster's bytes are bytes_algorithmic minus
                                       these (hqs: twice the planes plus the colour
                                       of the drawn points, minus these)          */

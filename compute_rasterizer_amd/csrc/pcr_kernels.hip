@@ -552,9 +552,14 @@ __device__ __forceinline__ bool rect_open(const void* __restrict__ buf, int widt
 // together, measured the same: the other waves of the SIMD already cover the
 // wait. row = i / tw as a multiply-high by magic = ceil(2^32 / tw): exact
 // because i < 2^13 and 2 <= tw <= 2^13 keep the error below 1/tw.
+//
+// The touched pixels are those whose key names one of the points [first, first
+// + np) just drawn: a pixel that still holds PCR_FB_CLEAR, or the key of
+// another point that tile_preload() found, is left without a load.
 template <int BLOCK>
 __device__ __forceinline__ void tile_flush(const unsigned long long* tile, unsigned long long* __restrict__ fb, int x0,
-                                           int y0, int tw, int n, uint32_t magic, uint32_t width, uint32_t* natom) {
+                                           int y0, int tw, int n, uint32_t magic, uint32_t width, uint32_t* natom,
+                                           uint32_t first, uint32_t np) {
     constexpr int F = 4;
     for (int i0 = threadIdx.x; i0 < n; i0 += F * BLOCK) {
         unsigned long long k[F], old[F];
@@ -563,6 +568,8 @@ __device__ __forceinline__ void tile_flush(const unsigned long long* tile, unsig
         for (int j = 0; j < F; j++) {
             const int i = i0 + j * BLOCK;
             k[j] = i < n ? tile[i] : PCR_FB_CLEAR;
+            const bool drawn = i < n && (uint32_t)k[j] - first < np;
+            if (!drawn) k[j] = PCR_FB_CLEAR;
             const uint32_t uy = __umulhi((uint32_t)i, magic), ux = (uint32_t)i - uy * (uint32_t)tw;
             pix[j] = (uint32_t)x0 + ux + ((uint32_t)y0 + uy) * width;
         }
@@ -700,44 +707,53 @@ struct QueueTake {
     }
 };
 
-// The groups of a batch that its tile may still need, and the words the
-// workgroup decides it with.
+// The words that a workgroup decides with what of a batch to draw.
 template <int BLOCK>
 struct GroupList {
-    uint32_t open[BLOCK / 64], closed[BLOCK / 64];   // per wave: threads with an open, a closed pixel
-    uint32_t n;                                      // groups in `live`
-    uint32_t skipped;                                // points of the others
-    uint32_t live[BLOCK];
+    uint32_t open[BLOCK / 64], closed[BLOCK / 64];   // per wave: threads with an open pixel, closed pixels
+    uint32_t skipped;                                // points of the hidden groups
     int4 part[BLOCK / 16];                           // batch_range: x0, y0, x1, y1 of 16 groups
     float part_w[BLOCK / 16];                        // and a depth none of their points undercuts
 };
 
 // Loads the framebuffer's keys over a rectangle of n pixels into the tile.
 // The tile then holds what the rectangle has at this moment: a point behind
-// it fails lds_min's first read, and the flush issues an atomic only for the
-// pixels that changed. Returns 0 when no pixel may take a point at depth wlo
+// it fails lds_min's first read. Returns 0 when no pixel may take a point at depth wlo
 // or beyond (the batch is hidden; rect_open has the reasons), 1 when some may,
-// 2 when also at least a quarter of the threads hold a pixel that may not.
+// 2 when also at least a quarter of them may not. (The test of the groups
+// then leaves out enough to pay: from half on, the overview below takes 1,160
+// us for 1,135, from three quarters on 1,245.)
 // Ends in a barrier.
 template <int BLOCK>
 __device__ __forceinline__ int tile_preload(unsigned long long* tile, const unsigned long long* __restrict__ fb, int x0,
                                             int y0, int tw, int n, uint32_t magic, uint32_t width, uint32_t wb,
                                             GroupList<BLOCK>& gl) {
-    bool open = false, closed = false;
-    for (int i = threadIdx.x; i < n; i += BLOCK) {
-        const uint32_t uy = __umulhi((uint32_t)i, magic), ux = (uint32_t)i - uy * (uint32_t)tw;
-        const unsigned long long k = fb[(uint32_t)x0 + ux + ((uint32_t)y0 + uy) * width];
-        tile[i] = k;
-        const bool o = (uint32_t)(k >> 32) >= wb;
-        open |= o;
-        closed |= !o;
+    bool open = false;
+    uint32_t closed = 0;   // of the wave
+    constexpr int F = 4;   // loads in flight per thread
+    for (int i0 = threadIdx.x; i0 < n; i0 += F * BLOCK) {
+        unsigned long long k[F];
+#pragma unroll
+        for (int j = 0; j < F; j++) {   // past the end: the last pixel again
+            const uint32_t i = (uint32_t)min(i0 + j * BLOCK, n - 1);
+            const uint32_t uy = __umulhi(i, magic), ux = i - uy * (uint32_t)tw;
+            k[j] = fb[(uint32_t)x0 + ux + ((uint32_t)y0 + uy) * width];
+        }
+#pragma unroll
+        for (int j = 0; j < F; j++) {
+            const int i = i0 + j * BLOCK;
+            if (i < n) tile[i] = k[j];
+            const bool o = (uint32_t)(k[j] >> 32) >= wb;
+            open |= o;
+            closed += (uint32_t)__popcll(__ballot(!o && i < n));
+        }
     }
-    const unsigned long long mo = __ballot(open), mc = __ballot(closed);
+    const unsigned long long mo = __ballot(open);
     if (__lane_id() == 0) {
         gl.open[threadIdx.x >> 6] = (uint32_t)__popcll(mo);
-        gl.closed[threadIdx.x >> 6] = (uint32_t)__popcll(mc);
+        gl.closed[threadIdx.x >> 6] = closed;
     }
-    if (threadIdx.x == 0) gl.n = gl.skipped = 0;
+    if (threadIdx.x == 0) gl.skipped = 0;
     __syncthreads();
     uint32_t no = 0, nc = 0;
 #pragma unroll
@@ -747,17 +763,20 @@ __device__ __forceinline__ int tile_preload(unsigned long long* tile, const unsi
     }
     no = __builtin_amdgcn_readfirstlane(no);
     nc = __builtin_amdgcn_readfirstlane(nc);
-    return no == 0 ? 0 : (nc * 4u >= (uint32_t)min(n, BLOCK) ? 2 : 1);
+    return no == 0 ? 0 : (nc * 4u >= (uint32_t)n ? 2 : 1);
 }
 
 // tile_loop() for an interior batch at the 10-bit level whose tile was
 // preloaded, without the groups of 64 points that lie behind the tile's
 // depths everywhere (VALU-bound: a point costs some 45 instructions, a
-// group's test about four points' worth): one thread tests one group's rectangle against the tile
-// (group_rect bounds where its points land and how near they are; the
-// reasoning is rect_open's), then 16 lanes draw each remaining group.
-// A group over more than kGroupTestPix pixels is drawn untested: its test
-// would cost more than its points.
+// group's test about four points' worth). Each wave takes every fourth group:
+// a lane tests one group's rectangle against the tile (group_rect bounds where
+// its points land and how near they are; the reasoning is rect_open's), and
+// the wave then draws the remaining groups, four at a time, 16 lanes each.
+// The waves need no list in LDS and no barrier for it, and the interleaving
+// shares out the hidden groups, which lie together. A group over more than
+// kGroupTestPix pixels is drawn untested: its test would cost more than its
+// points.
 constexpr int kGroupTestPix = 64;
 template <int BLOCK, bool NT>
 __device__ __forceinline__ void tile_groups(const Decode& d, const uint32_t* __restrict__ lo,
@@ -765,16 +784,13 @@ __device__ __forceinline__ void tile_groups(const Decode& d, const uint32_t* __r
                                             const Proj& pj, GroupSlack slack, unsigned long long* __restrict__ fb,
                                             unsigned long long* tile, int x0, int y0, int tw, int th, uint32_t* natom,
                                             GroupList<BLOCK>& gl) {
+    constexpr uint32_t kWaves = BLOCK / 64;
     const uint32_t first = h.first_point, np = h.num_points;
     const uint32_t lead = first & 3u, ng = groups_of(first, np), nq = (np + lead + 3u) >> 2;
     const u32x4* lo4 = reinterpret_cast<const u32x4*>(lo + (first - lead));
-    for (uint32_t g0 = 0; g0 < ng; g0 += BLOCK) {
-        if (g0) {   // the list of the last BLOCK groups has been drawn
-            __syncthreads();
-            if (threadIdx.x == 0) gl.n = 0;
-            __syncthreads();
-        }
-        const uint32_t g = g0 + threadIdx.x;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = __lane_id(), row = lane >> 4;
+    for (uint32_t g0 = wave; g0 < ng; g0 += BLOCK) {
+        const uint32_t g = g0 + lane * kWaves;
         bool live = g < ng;
         if (live) {
             const GroupRect r = group_rect(box[g], 2, d, v.transform, v.width, v.height, slack.px, slack.w);
@@ -793,18 +809,18 @@ __device__ __forceinline__ void tile_groups(const Decode& d, const uint32_t* __r
                 lds_add32(&gl.skipped, end - beg);
             }
         }
-        const unsigned long long m = __ballot(live);
-        uint32_t base = 0;
-        if (__lane_id() == 0 && m)
-            base = __hip_atomic_fetch_add((lds_u32*)&gl.n, (uint32_t)__popcll(m), __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_WORKGROUP);
-        base = __builtin_amdgcn_readfirstlane(base);
-        if (live) gl.live[base + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull))] = g;
-        __syncthreads();
-        const uint32_t n = __builtin_amdgcn_readfirstlane(gl.n);
-        for (uint32_t j = threadIdx.x >> 4; j < n; j += BLOCK / 16) {
-            const uint32_t q = gl.live[j] * (kGroupPoints / 4) + (threadIdx.x & 15u);
-            if (q >= nq) continue;
+        unsigned long long m = __ballot(live);
+        while (m) {
+            // the row's group: the row-th of the lowest four left
+            uint32_t sel = 64;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++) {
+                const uint32_t bit = m ? (uint32_t)__builtin_ctzll(m) : 64u;
+                m &= m - 1ull;
+                if (row == k) sel = bit;
+            }
+            const uint32_t q = (g0 + sel * kWaves) * (kGroupPoints / 4) + (lane & 15u);
+            if (sel == 64u || q >= nq) continue;
             const u32x4 a = ld_plane<NT>(lo4 + q);
             const uint32_t base = q * 4u - lead;
             tile_point<2, true, true>(d, a.x, 0u, 0u, base + 0, np, first, pj, fb, tile, x0, y0, tw, th, natom);
@@ -865,7 +881,8 @@ __device__ __forceinline__ uint32_t tiled_batch(uint32_t bi, int level, const pc
         __syncthreads();
         tile_dispatch<BLOCK, true, NT>(level, d, lo, med, hi, h, pj, fb, tile, x0, y0, tw, th, natom, interior);
         __syncthreads();
-        tile_flush<BLOCK>(tile, fb, x0, y0, tw, n, row_magic(tw), (uint32_t)v.width, natom);
+        tile_flush<BLOCK>(tile, fb, x0, y0, tw, n, row_magic(tw), (uint32_t)v.width, natom, h.first_point,
+                          h.num_points);
     } else {
         tile_dispatch<BLOCK, false, NT>(level, d, lo, med, hi, h, pj, fb, nullptr, 0, 0, 0, 0, natom);
     }
@@ -1017,7 +1034,8 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
                 }
                 __syncthreads();
                 if (tests) skipped += gl.skipped;
-                tile_flush<BLOCK>(tile, fb, x0, y0, tw, n, magic, (uint32_t)v.width, natom);
+                tile_flush<BLOCK>(tile, fb, x0, y0, tw, n, magic, (uint32_t)v.width, natom, h.first_point,
+                                  h.num_points);
             } else {
                 tile_dispatch<BLOCK, false, true>(level, d, lo, med, hi, h, pj, fb, nullptr, 0, 0, 0, 0, natom);
             }
@@ -1231,9 +1249,11 @@ __device__ __forceinline__ bool raster_pair_batch(uint32_t bi, int level, const 
     __syncthreads();
     // each view's flush, as in tiled_batch
     if (a.draw)
-        tile_flush<BLOCK>(a.tile, a.fb, a.x0, a.y0, a.tw, a.tw * a.th, row_magic(a.tw), (uint32_t)a.pj.w, natom);
+        tile_flush<BLOCK>(a.tile, a.fb, a.x0, a.y0, a.tw, a.tw * a.th, row_magic(a.tw), (uint32_t)a.pj.w, natom,
+                          h.first_point, h.num_points);
     if (c.draw)
-        tile_flush<BLOCK>(c.tile, c.fb, c.x0, c.y0, c.tw, c.tw * c.th, row_magic(c.tw), (uint32_t)c.pj.w, natom);
+        tile_flush<BLOCK>(c.tile, c.fb, c.x0, c.y0, c.tw, c.tw * c.th, row_magic(c.tw), (uint32_t)c.pj.w, natom,
+                          h.first_point, h.num_points);
     return true;
 }
 

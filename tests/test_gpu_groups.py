@@ -134,4 +134,8 @@ def test_grouped_raster_equals_oracle(ctx, n, size, shift, shuffle, tile_px, blo
                                             clear_before=False), fb)
             assert np.array_equal(fb.keys(), ref) and ctx.stats().atomics_issued == 0
             fb.close()
+        fb = ctx.framebuffer(v.width, v.height)
+        ctx.render(cloud, v, pcr.params(pcr.MODE_LAS), fb)
+        assert np.array_equal(fb.keys(), ref) and ctx.stats().points_occluded == 0
+        fb.close()
     cloud.close()

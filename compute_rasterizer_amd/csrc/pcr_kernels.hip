@@ -893,9 +893,9 @@ __device__ __forceinline__ uint32_t tiled_batch(uint32_t bi, int level, const pc
 // g0 on, into gl.part: one thread bounds one group, and the 16 lanes of a part
 // join theirs. A part outside the image has an empty rectangle; one without a
 // bound has a rectangle that fits no tile. Ends in a barrier.
-template <int BLOCK>
+template <int BLOCK, class List>
 __device__ __forceinline__ void batch_parts(const uint2* __restrict__ box, uint32_t g0, uint32_t ng, int level,
-                                            const Decode& d, const pcr_view& v, GroupSlack slack, GroupList<BLOCK>& gl) {
+                                            const Decode& d, const pcr_view& v, GroupSlack slack, List& gl) {
     constexpr int kOut = 1 << 20;   // beyond any pixel
     int x0 = kOut, y0 = kOut, x1 = -1, y1 = -1;
     float w = 3e38f;
@@ -924,6 +924,52 @@ __device__ __forceinline__ void batch_parts(const uint2* __restrict__ box, uint3
         gl.part_w[threadIdx.x >> 4] = fmaxf(w, 0.0f);
     }
     __syncthreads();
+}
+
+// The next run of parts of a batch, from group g on (a multiple of 16 groups;
+// moved past the run): as many parts as have a joint rectangle of at most CAP
+// pixels, or a single part.
+struct BatchRun {
+    int x0, y0, tw, th;    // tw <= 0: outside the image
+    float w;               // a depth none of its points undercuts
+    uint32_t first, num;   // its points
+};
+template <int CAP>
+__device__ __forceinline__ bool run_fits(int w, int h) {
+    return w >= 2 && w <= CAP && h <= CAP && w * h <= CAP;
+}
+template <int BLOCK, int CAP, class List>
+__device__ __forceinline__ BatchRun next_run(const uint2* __restrict__ box, uint32_t& g, uint32_t ng, const pcr_batch& h,
+                                             uint32_t first, uint32_t np, uint32_t lead, int level, const pcr_view& v,
+                                             float wnear, List& gl) {
+    const uint32_t p0 = (g & (BLOCK - 1u)) >> 4;
+    if (p0 == 0)
+        batch_parts<BLOCK>(box, g, ng, level, make_decode(level, h.min, h.max), v,
+                           group_slack(v.transform, h.min, h.max, v.width, v.height, wnear), gl);
+    const uint32_t left = min((ng - g + 15u) >> 4, BLOCK / 16u - p0);
+    int r[4] = {gl.part[p0].x, gl.part[p0].y, gl.part[p0].z, gl.part[p0].w};
+    float w = gl.part_w[p0];
+    uint32_t n = 1;
+    for (; n < left; n++) {   // join the next part while the rectangle fits
+        const int4 q = gl.part[p0 + n];
+        const int a0 = min(r[0], q.x), a1 = min(r[1], q.y), a2 = max(r[2], q.z), a3 = max(r[3], q.w);
+        if (a2 >= 0 && !run_fits<CAP>(max(a2 - a0 + 1, 2), a3 - a1 + 1)) break;
+        r[0] = a0; r[1] = a1; r[2] = a2; r[3] = a3;
+        w = fminf(w, gl.part_w[p0 + n]);
+    }
+    n = __builtin_amdgcn_readfirstlane(n);
+    BatchRun run;
+    run.x0 = __builtin_amdgcn_readfirstlane(r[0]);
+    run.y0 = __builtin_amdgcn_readfirstlane(r[1]);
+    run.tw = __builtin_amdgcn_readfirstlane(r[2]) - run.x0 + 1;
+    run.th = __builtin_amdgcn_readfirstlane(r[3]) - run.y0 + 1;
+    run.w = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(w)));
+    const uint32_t w0 = g * kGroupPoints, w1 = (g + n * 16u) * kGroupPoints;
+    const uint32_t o0 = w0 > lead ? w0 - lead : 0u, o1 = min(w1 - lead, np);
+    run.first = first + o0;
+    run.num = o1 - o0;
+    g += n * 16u;
+    return run;
 }
 
 // One batch of the tiled raster for a cloud with group bounds; `bi` and
@@ -965,39 +1011,17 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
     float wlo, wnear;
     bool use = screen_rect(v.transform, h.min, h.max, v.width, v.height, x0, y0, x1, y1, &interior, &wlo, &wnear);
     int tw = x1 - x0 + 1, th = y1 - y0 + 1;
-    const auto fits = [](int w, int hh) { return w >= 2 && w <= TILE_PIX && hh <= TILE_PIX && w * hh <= TILE_PIX; };
+    const auto fits = [](int w, int hh) { return run_fits<TILE_PIX>(w, hh); };
     const bool parted = use && !fits(tw, th) && wnear > 0.0f;
     const uint32_t first = h.first_point, np = h.num_points, lead = first & 3u, ng = groups_of(first, np);
     uint32_t skipped = 0, g = 0;   // g: the first group not yet drawn
     for (;;) {
         bool tests = occl && wlo > 0.0f;
         if (parted) {
-            const uint32_t p0 = (g & (BLOCK - 1u)) >> 4;
-            if (p0 == 0)
-                batch_parts<BLOCK>(box, g, ng, level, make_decode(level, h.min, h.max), v,
-                                   group_slack(v.transform, h.min, h.max, v.width, v.height, wnear), gl);
-            const uint32_t left = min((ng - g + 15u) >> 4, BLOCK / 16u - p0);
-            int r[4] = {gl.part[p0].x, gl.part[p0].y, gl.part[p0].z, gl.part[p0].w};
-            float w = gl.part_w[p0];
-            uint32_t n = 1;
-            for (; n < left; n++) {   // join the next part while the rectangle fits
-                const int4 q = gl.part[p0 + n];
-                const int a0 = min(r[0], q.x), a1 = min(r[1], q.y), a2 = max(r[2], q.z), a3 = max(r[3], q.w);
-                if (a2 >= 0 && !fits(max(a2 - a0 + 1, 2), a3 - a1 + 1)) break;
-                r[0] = a0; r[1] = a1; r[2] = a2; r[3] = a3;
-                w = fminf(w, gl.part_w[p0 + n]);
-            }
-            n = __builtin_amdgcn_readfirstlane(n);
-            x0 = __builtin_amdgcn_readfirstlane(r[0]);
-            y0 = __builtin_amdgcn_readfirstlane(r[1]);
-            tw = __builtin_amdgcn_readfirstlane(r[2]) - x0 + 1;
-            th = __builtin_amdgcn_readfirstlane(r[3]) - y0 + 1;
-            wlo = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(w)));
-            const uint32_t w0 = g * kGroupPoints, w1 = (g + n * 16u) * kGroupPoints;
-            const uint32_t o0 = w0 > lead ? w0 - lead : 0u, o1 = min(w1 - lead, np);
-            h.first_point = first + o0;
-            h.num_points = o1 - o0;
-            g += n * 16u;
+            const BatchRun r = next_run<BLOCK, TILE_PIX>(box, g, ng, h, first, np, lead, level, v, wnear, gl);
+            x0 = r.x0; y0 = r.y0; tw = r.tw; th = r.th; wlo = r.w;
+            h.first_point = r.first;
+            h.num_points = r.num;
             tests = occl;
             use = fits(tw, th);
             if (tw <= 0) {   // outside the image
@@ -1548,13 +1572,13 @@ __device__ __forceinline__ void hqs_tile_dispatch(int level, const Decode& d, co
                                                 tdepth, tacc, tb);
 }
 
-// Pass 2 keeps 20 B per tile pixel; its tile holds 24 pixels fewer than
+// Pass 2 keeps 20 B per tile pixel; its tile holds 48 pixels fewer than
 // TILE_PIX so that with the kernels' other shared words (and the block-wide
 // OR of the occlusion test) four 256-thread workgroups still fit a CU's
 // 160 KB of LDS at TILE_PIX = 2048.
 template <int PASS, int TILE_PIX>
 struct HqsTile {
-    static constexpr int kCap = PASS == 1 ? TILE_PIX - 24 : TILE_PIX;
+    static constexpr int kCap = PASS == 1 ? TILE_PIX - 48 : TILE_PIX;
     uint32_t depth[kCap];
     unsigned long long acc[PASS == 1 ? 2 * kCap : 1];
 };
@@ -1583,15 +1607,108 @@ __device__ __forceinline__ void hqs_depth_flush(const uint32_t* tdepth, uint32_t
         hqs_depth(depth, (uint32_t)x0 + ux + (by0 + uy) * width, t);
     }
 }
+// `closed`: takes, per wave, the pixels that a point at depth wlo or beyond
+// does not reach (depth_open<2>).
 template <int BLOCK>
 __device__ __forceinline__ void hqs_sums_preload(uint32_t* tdepth, unsigned long long* tacc,
                                                  const uint32_t* __restrict__ depth, int x0, uint32_t by0, int tw,
-                                                 int n, uint32_t magic, uint32_t width) {
+                                                 int n, uint32_t magic, uint32_t width, float wlo, uint32_t* closed) {
+    uint32_t c = 0;
     for (int i = threadIdx.x; i < n; i += BLOCK) {
         const uint32_t uy = __umulhi((uint32_t)i, magic), ux = (uint32_t)i - uy * (uint32_t)tw;
-        tdepth[i] = depth[(uint32_t)x0 + ux + (by0 + uy) * width];
+        const uint32_t d = depth[(uint32_t)x0 + ux + (by0 + uy) * width];
+        tdepth[i] = d;
         tacc[2 * i] = 0ull;
         tacc[2 * i + 1] = 0ull;
+        c += (uint32_t)__popcll(__ballot(!(__uint_as_float(d) * 1.01f >= wlo)));
+    }
+    if (__lane_id() == 0) closed[threadIdx.x >> 6] = c;   // a wave's first lane makes all its rounds
+}
+
+// Group test of pass 2: the final depths are known, so 0.6 of the groups of a
+// dense cloud are behind them. Tests the group's rectangle against
+// a view's tile; the reasoning is rect_open's (kind 2).
+constexpr uint32_t kHqsGateDiv = 8;   // from this share of closed pixels on the groups are tested
+template <int BLOCK>
+struct HqsGroups {
+    uint32_t closed[2][BLOCK / 64];   // per view of a pair and wave
+    uint32_t skipped;                 // points of the groups left out
+    int4 part[BLOCK / 16];            // batch_parts()
+    float part_w[BLOCK / 16];
+    __device__ __forceinline__ bool many(int view, int n) const {
+        uint32_t c = 0;
+#pragma unroll
+        for (int w = 0; w < BLOCK / 64; w++) c += closed[view][w];
+        return __builtin_amdgcn_readfirstlane(c) * kHqsGateDiv >= (uint32_t)n;
+    }
+};
+__device__ __forceinline__ bool hqs_group_open(uint2 box, const Decode& d, const pcr_view& v, GroupSlack slack,
+                                               const uint32_t* tdepth, int x0, int y0, int tw, int th) {
+    const GroupRect r = group_rect(box, 2, d, v.transform, v.width, v.height, slack.px, slack.w);
+    const int rx0 = max(r.x0 - x0, 0), ry0 = max(r.y0 - y0, 0), rx1 = min(r.x1 - x0, tw - 1),
+              ry1 = min(r.y1 - y0, th - 1);
+    const int rw = rx1 - rx0 + 1, rh = ry1 - ry0 + 1;
+    if (r.wild || rw <= 0 || rh <= 0 || rw > kGroupTestPix || rh > kGroupTestPix || rw * rh > kGroupTestPix) return true;
+    bool open = false;
+    for (int y = ry0; y <= ry1 && !open; y++)
+        for (int x = rx0; x <= rx1 && !open; x++) open = __uint_as_float(tdepth[y * tw + x]) * 1.01f >= r.w;
+    return open;
+}
+// The eight lowest set bits of m, one per 8 lanes of the wave (64: none left).
+__device__ __forceinline__ uint32_t take8(unsigned long long& m) {
+    uint32_t sel = 64;
+    const uint32_t row = __lane_id() >> 3;
+#pragma unroll
+    for (uint32_t k = 0; k < 8; k++) {
+        const uint32_t bit = m ? (uint32_t)__builtin_ctzll(m) : 64u;
+        m &= m - 1ull;
+        if (row == k) sel = bit;
+    }
+    return sel;
+}
+__device__ __forceinline__ uint32_t group_points(uint32_t g, uint32_t lead, uint32_t np) {
+    return min((g + 1) * kGroupPoints, np + lead) - max(g * kGroupPoints, lead);
+}
+
+// Pass 2 of an interior batch at the 10-bit level in one band, without the
+// hidden groups, each wave every fourth group as in tile_groups(). Eight lanes
+// draw a group, eight consecutive points a lane, the runs that PendingSums
+// joins elsewhere.
+template <int BLOCK, bool NT>
+__device__ __forceinline__ void hqs2_groups(const Decode& d, const uint32_t* __restrict__ lo,
+                                            const uint32_t* __restrict__ rgba, const uint2* __restrict__ box,
+                                            const pcr_batch& h, const pcr_view& v, const Proj& pj, GroupSlack slack,
+                                            uint32_t* __restrict__ depth, uint32_t* __restrict__ acc, uint32_t* tdepth,
+                                            unsigned long long* tacc, const TileBand& tb, HqsGroups<BLOCK>& hg) {
+    constexpr uint32_t kWaves = BLOCK / 64;
+    const uint32_t first = h.first_point, np = h.num_points;
+    const uint32_t lead = first & 3u, ng = groups_of(first, np), nq = (np + lead + 3u) >> 2;
+    const u32x4* lo4 = reinterpret_cast<const u32x4*>(lo + (first - lead));
+    const u32x4* c4 = reinterpret_cast<const u32x4*>(rgba + (first - lead));
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = __lane_id();
+    for (uint32_t g0 = wave; g0 < ng; g0 += BLOCK) {
+        const uint32_t g = g0 + lane * kWaves;
+        bool live = g < ng;
+        if (live && !hqs_group_open(box[g], d, v, slack, tdepth, tb.x0, tb.y0, tb.tw, tb.th)) {
+            live = false;
+            lds_add32(&hg.skipped, group_points(g, lead, np));
+        }
+        unsigned long long m = __ballot(live);
+        while (m) {
+            const uint32_t sel = take8(m), q0 = (g0 + sel * kWaves) * (kGroupPoints / 4) + (lane & 7u) * 2u;
+            if (sel == 64u || q0 >= nq) continue;
+            const bool two = q0 + 1u < nq;
+            const u32x4 z = u32x4{0, 0, 0, 0};
+            const u32x4 a0 = ld_plane<NT>(lo4 + q0), k0 = ld_plane<NT>(c4 + q0);
+            const u32x4 a1 = two ? ld_plane<NT>(lo4 + q0 + 1) : z, k1 = two ? ld_plane<NT>(c4 + q0 + 1) : z;
+            PendingSums pend;
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                hqs_tile_point<1, 2, true, true>(d, j < 4 ? a0[j & 3] : a1[j & 3], 0u, 0u, j < 4 ? k0[j & 3] : k1[j & 3],
+                                                 q0 * 4u - lead + (uint32_t)j, np, pj, depth, acc, tdepth, tacc, tb,
+                                                 pend);
+            pending_flush(pend, tacc);
+        }
     }
 }
 template <int BLOCK>
@@ -1614,20 +1731,22 @@ __device__ __forceinline__ uint32_t hqs_tiled_batch(uint32_t bi, int level, cons
                                                 const pcr_view& v, uint32_t* __restrict__ depth,
                                                 uint32_t* __restrict__ acc, uint32_t* tdepth,
                                                 unsigned long long* tacc, bool occl, uint32_t part = 0,
-                                                uint32_t nparts = 1) {
+                                                uint32_t nparts = 1, const uint2* __restrict__ box = nullptr,
+                                                HqsGroups<BLOCK>* hg = nullptr) {
     const pcr_batch h = b[bi];
     pcr_batch hp = h;   // the points this item draws; the tile and band choices follow the whole batch
     if (nparts > 1) {
         batch_part(hp, part, nparts);
         if (hp.num_points == 0) return 0;
+        if (box) box += ((hp.first_point & ~3u) - (h.first_point & ~3u)) / kGroupPoints;   // parts are whole groups
     }
     const Decode d = make_decode(level, h.min, h.max);
     const Proj pj = make_proj(v.transform, v.width, v.height);
     int x0 = 0, y0 = 0, x1 = -1, y1 = -1;
     bool interior;
-    float wlo;
+    float wlo, wnear;
     const bool on_screen = screen_rect(v.transform, h.min, h.max, v.width, v.height, x0, y0, x1, y1, &interior,
-                                       &wlo);
+                                       &wlo, &wnear);
     const int tw = x1 - x0 + 1, th = y1 - y0 + 1;
     // pass 1: behind every depth already drawn over the rectangle; pass 2:
     // behind 1.01x every final depth there (rect_open)
@@ -1638,6 +1757,53 @@ __device__ __forceinline__ uint32_t hqs_tiled_batch(uint32_t bi, int level, cons
     // one-column rectangles draw directly, as in tiled_batch (tw >= 2 keeps
     // the row split's ceil(2^32 / tw) within 32 bits)
     const bool fits = on_screen && tw >= 2 && tw <= cap && h.num_points <= kHqsTileMaxPoints;
+    if (box && on_screen && wnear > 0.0f && !(fits && run_fits<cap>(tw, th))) {
+        // A rectangle larger than the tile, in runs of parts as in
+        // grouped_batch(): bands project every point once per band, and the
+        // direct path of pass 2 makes two atomics per point. Without the runs
+        // the passes over a 500M-point city (10,320 batches drawn) take 335 and
+        // 626 us, with them 214 and 355; over 350 octree nodes 78 and 123, and
+        // 57 and 99.
+        const uint32_t first = hp.first_point, np = hp.num_points, lead = first & 3u, ng = groups_of(first, np);
+        uint32_t skipped = 0;
+        for (uint32_t g = 0; g < ng;) {
+            const uint32_t gr = g;
+            const BatchRun r = next_run<BLOCK, cap>(box, g, ng, h, first, np, lead, level, v, wnear, *hg);
+            if (r.tw <= 0) continue;   // outside the image
+            hp.first_point = r.first;
+            hp.num_points = r.num;
+            if (!run_fits<cap>(r.tw, r.th)) {
+                const TileBand none{0, 0, 0, 0, 0, 0, true};
+                hqs_tile_dispatch<BLOCK, PASS, false, NT>(level, d, lo, med, hi, rgba, hp, pj, depth, acc, nullptr,
+                                                          nullptr, none);
+                continue;
+            }
+            const int n = r.tw * r.th;
+            const uint32_t magic = row_magic(r.tw), width = (uint32_t)v.width;
+            if (PASS == 0) {
+                for (int i = threadIdx.x; i < n; i += BLOCK) tdepth[i] = PCR_DEPTH_CLEAR;
+            } else {
+                if (threadIdx.x == 0) hg->skipped = 0;
+                hqs_sums_preload<BLOCK>(tdepth, tacc, depth, r.x0, (uint32_t)r.y0, r.tw, n, magic, width, r.w,
+                                        hg->closed[0]);
+            }
+            __syncthreads();
+            const TileBand tb{r.x0, r.y0, r.tw, r.th, 0, r.th, true};
+            if (PASS == 1 && occl && interior && level >= 2 && hg->many(0, n))
+                hqs2_groups<BLOCK, NT>(d, lo, rgba, box + gr, hp, v, pj,
+                                       group_slack(v.transform, h.min, h.max, v.width, v.height, wnear), depth, acc,
+                                       tdepth, tacc, tb, *hg);
+            else
+                hqs_tile_dispatch<BLOCK, PASS, true, NT>(level, d, lo, med, hi, rgba, hp, pj, depth, acc, tdepth, tacc,
+                                                         tb, interior);
+            __syncthreads();
+            if (PASS == 1) skipped += hg->skipped;
+            if (PASS == 0) hqs_depth_flush<BLOCK>(tdepth, depth, r.x0, (uint32_t)r.y0, r.tw, n, magic, width);
+            else hqs_sums_flush<BLOCK>(tacc, acc, r.x0, (uint32_t)r.y0, r.tw, n, magic, width);
+            __syncthreads();   // the tile and the count are reused by the next run
+        }
+        return skipped;
+    }
     const int bh = fits ? min(th, cap / tw) : 1;    // rows per band
     const int nbands = fits ? (th + bh - 1) / bh : 0;
     // bands pay when the batch is dense (a point or more per rectangle pixel,
@@ -1650,6 +1816,7 @@ __device__ __forceinline__ uint32_t hqs_tiled_batch(uint32_t bi, int level, cons
         return 0;
     }
     const uint32_t magic = row_magic(tw), width = (uint32_t)v.width;
+    if (PASS == 1 && threadIdx.x == 0) hg->skipped = 0;
     for (int k = 0; k < nbands; k++) {
         const int boff = k * bh, rows = min(bh, th - boff);
         const int n = tw * rows;
@@ -1658,16 +1825,21 @@ __device__ __forceinline__ uint32_t hqs_tiled_batch(uint32_t bi, int level, cons
         if (PASS == 0)
             for (int i = threadIdx.x; i < n; i += BLOCK) tdepth[i] = PCR_DEPTH_CLEAR;
         else
-            hqs_sums_preload<BLOCK>(tdepth, tacc, depth, x0, by0, tw, n, magic, width);
+            hqs_sums_preload<BLOCK>(tdepth, tacc, depth, x0, by0, tw, n, magic, width, wlo, hg->closed[0]);
         __syncthreads();
         const TileBand tb{x0, y0, tw, th, boff, rows, k == 0};
-        hqs_tile_dispatch<BLOCK, PASS, true, NT>(level, d, lo, med, hi, rgba, hp, pj, depth, acc, tdepth, tacc, tb,
-                                                 interior);
+        if (PASS == 1 && occl && box && wlo > 0.0f && level >= 2 && nbands == 1 && hg->many(0, n))
+            hqs2_groups<BLOCK, NT>(d, lo, rgba, box, hp, v, pj,
+                                   group_slack(v.transform, h.min, h.max, v.width, v.height, wlo), depth, acc, tdepth,
+                                   tacc, tb, *hg);
+        else
+            hqs_tile_dispatch<BLOCK, PASS, true, NT>(level, d, lo, med, hi, rgba, hp, pj, depth, acc, tdepth, tacc, tb,
+                                                     interior);
         __syncthreads();
         if (PASS == 0) hqs_depth_flush<BLOCK>(tdepth, depth, x0, by0, tw, n, magic, width);
         else hqs_sums_flush<BLOCK>(tacc, acc, x0, by0, tw, n, magic, width);
     }
-    return 0;
+    return PASS == 1 ? hg->skipped : 0;
 }
 
 // hqs pass 1 of one batch for a pair of views at once, the next two views a
@@ -1818,6 +1990,49 @@ __device__ __forceinline__ void hqs2_view_point(const float p[3], uint32_t color
     hqs_accum(pv.depth, pv.acc, (uint32_t)ix + (uint32_t)iy * (uint32_t)pv.pj.w, dep, color);
 }
 
+// hqs2_pair_loop() at the 10-bit level without the groups hidden in both views;
+// a group is drawn in the views where it is not hidden.
+template <int BLOCK, bool NT>
+__device__ __forceinline__ void hqs2_pair_groups(const Decode& d, const uint32_t* __restrict__ lo,
+                                                 const uint32_t* __restrict__ rgba, const uint2* __restrict__ box,
+                                                 uint32_t first, uint32_t np, const pcr_view& va, GroupSlack sa,
+                                                 const Pair2View& a, const pcr_view& vc, GroupSlack sc,
+                                                 const Pair2View& c) {
+    constexpr uint32_t kWaves = BLOCK / 64;
+    const uint32_t lead = first & 3u, ng = groups_of(first, np), nq = (np + lead + 3u) >> 2;
+    const u32x4* lo4 = reinterpret_cast<const u32x4*>(lo + (first - lead));
+    const u32x4* c4 = reinterpret_cast<const u32x4*>(rgba + (first - lead));
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = __lane_id();
+    for (uint32_t g0 = wave; g0 < ng; g0 += BLOCK) {
+        const uint32_t g = g0 + lane * kWaves;
+        bool la = g < ng && a.draw, lc = g < ng && c.draw;
+        if (la) la = hqs_group_open(box[g], d, va, sa, a.tdepth, a.tb.x0, a.tb.y0, a.tb.tw, a.tb.th);
+        if (lc) lc = hqs_group_open(box[g], d, vc, sc, c.tdepth, c.tb.x0, c.tb.y0, c.tb.tw, c.tb.th);
+        const unsigned long long ma = __ballot(la), mc = __ballot(lc);
+        unsigned long long m = ma | mc;
+        while (m) {
+            const uint32_t sel = take8(m), q0 = (g0 + sel * kWaves) * (kGroupPoints / 4) + (lane & 7u) * 2u;
+            if (sel == 64u || q0 >= nq) continue;
+            const bool da = (ma >> sel) & 1ull, dc = (mc >> sel) & 1ull;
+            for (uint32_t q = q0; q < min(q0 + 2u, nq); q++) {
+                const u32x4 w = ld_plane<NT>(lo4 + q), col = ld_plane<NT>(c4 + q);
+                const uint32_t base = q * 4u - lead;
+                PendingSums pa, pc;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (base + (uint32_t)j >= np) continue;
+                    float p[3];
+                    decode<2>(d, w[j], 0u, 0u, p);
+                    if (da) hqs2_view_point(p, col[j], a, pa);
+                    if (dc) hqs2_view_point(p, col[j], c, pc);
+                }
+                pending_flush(pa, a.tacc);
+                pending_flush(pc, c.tacc);
+            }
+        }
+    }
+}
+
 template <int BLOCK, int LC, bool NT>
 __device__ __forceinline__ void hqs2_pair_loop(const Decode& d, const uint32_t* __restrict__ lo,
                                                const uint32_t* __restrict__ med, const uint32_t* __restrict__ hi,
@@ -1858,10 +2073,14 @@ __device__ __forceinline__ bool hqs2_pair_batch(uint32_t bi, int level, const pc
                                                 uint32_t* __restrict__ acc_a, const pcr_view& vb,
                                                 uint32_t* __restrict__ depth_b, uint32_t* __restrict__ acc_b,
                                                 uint32_t* tdepth, unsigned long long* tacc, bool occl, uint32_t part,
-                                                uint32_t nparts) {
+                                                uint32_t nparts, const uint2* __restrict__ box,
+                                                HqsGroups<BLOCK>& hg) {
     const pcr_batch h = b[bi];
     pcr_batch hp = h;   // as in hqs_tiled_batch: the points this item draws
-    if (nparts > 1) batch_part(hp, part, nparts);
+    if (nparts > 1) {
+        batch_part(hp, part, nparts);
+        if (box) box += ((hp.first_point & ~3u) - (h.first_point & ~3u)) / kGroupPoints;
+    }
     int ax0 = 0, ay0 = 0, ax1 = -1, ay1 = -1, bx0 = 0, by0 = 0, bx1 = -1, by1 = -1;
     bool ai, bi_;
     float awlo, bwlo;
@@ -1886,11 +2105,18 @@ __device__ __forceinline__ bool hqs2_pair_batch(uint32_t bi, int level, const pc
     // each drawing view's final depths into its half, its sums cleared
     const uint32_t am = row_magic(atw), cm = row_magic(btw);
     if (a.draw)
-        hqs_sums_preload<BLOCK>(a.tdepth, a.tacc, depth_a, ax0, (uint32_t)ay0, atw, atw * ath, am, (uint32_t)va.width);
+        hqs_sums_preload<BLOCK>(a.tdepth, a.tacc, depth_a, ax0, (uint32_t)ay0, atw, atw * ath, am, (uint32_t)va.width,
+                                awlo, hg.closed[0]);
     if (c.draw)
-        hqs_sums_preload<BLOCK>(c.tdepth, c.tacc, depth_b, bx0, (uint32_t)by0, btw, btw * bth, cm, (uint32_t)vb.width);
+        hqs_sums_preload<BLOCK>(c.tdepth, c.tacc, depth_b, bx0, (uint32_t)by0, btw, btw * bth, cm, (uint32_t)vb.width,
+                                bwlo, hg.closed[1]);
     __syncthreads();
-    if (level == 0) hqs2_pair_loop<BLOCK, 0, NT>(d, lo, med, hi, rgba, hp.first_point, hp.num_points, a, c);
+    if (level >= 2 && occl && box && awlo > 0.0f && bwlo > 0.0f &&
+        (!a.draw || hg.many(0, atw * ath)) && (!c.draw || hg.many(1, btw * bth)))
+        hqs2_pair_groups<BLOCK, NT>(d, lo, rgba, box, hp.first_point, hp.num_points, va,
+                                    group_slack(va.transform, h.min, h.max, va.width, va.height, awlo), a, vb,
+                                    group_slack(vb.transform, h.min, h.max, vb.width, vb.height, bwlo), c);
+    else if (level == 0) hqs2_pair_loop<BLOCK, 0, NT>(d, lo, med, hi, rgba, hp.first_point, hp.num_points, a, c);
     else if (level == 1) hqs2_pair_loop<BLOCK, 1, NT>(d, lo, med, hi, rgba, hp.first_point, hp.num_points, a, c);
     else hqs2_pair_loop<BLOCK, 2, NT>(d, lo, med, hi, rgba, hp.first_point, hp.num_points, a, c);
     __syncthreads();
@@ -1915,7 +2141,10 @@ void k_hqs_tiled(const pcr_batch* __restrict__ b,
                  const uint32_t* __restrict__ hi,
                  const uint32_t* __restrict__ rgba, pcr_view v,
                  uint32_t* __restrict__ depth,
-                 uint32_t* __restrict__ acc, int occl, uint32_t nb) {
+                 uint32_t* __restrict__ acc, int occl, uint32_t nb,
+                 const uint2* __restrict__ gbox,
+                 const uint32_t* __restrict__ gbase) {
+    __shared__ HqsGroups<BLOCK> hg;
     __shared__ HqsTile<PASS, TILE_PIX> tile;
     __shared__ uint32_t s_item;
     uint32_t* head = PASS == 0 ? &st->queue_head : &st->queue_head2;
@@ -1935,11 +2164,17 @@ void k_hqs_tiled(const pcr_batch* __restrict__ b,
         const int level = __builtin_amdgcn_readfirstlane(levels[bi]);
         const uint32_t skipped = hqs_tiled_batch<BLOCK, TILE_PIX, PASS, true>(bi, level, b, lo, med, hi, rgba, v,
                                                                               depth, acc, tile.depth, tile.acc,
-                                                                              occl != 0, part, nparts);
+                                                                              occl != 0, part, nparts,
+                                                                              gbox ? gbox + gbase[bi] : nullptr,
+                                                                              &hg);
         if (threadIdx.x == 0 && skipped) {
             s_occ_points += skipped;
             s_occ_bytes += (4ull * planes_for_level(level) + (PASS == 1 ? 4ull : 0ull)) * skipped;
-            s_occ_batches += part == 0;
+            if (part == 0) {   // as in k_raster_tiled
+                pcr_batch h = b[bi];
+                if (nparts > 1) batch_part(h, 0, nparts);
+                s_occ_batches += skipped == h.num_points;
+            }
         }
         __syncthreads();   // s_item and the tile are reused by the next item
     }
@@ -1966,7 +2201,8 @@ static void hqs_tiled_t(hipStream_t s, const pcr_cloud* c, const pcr_view& v, Fr
     if (grid > (uint64_t)c->num_batches * kMaxParts) grid = (uint64_t)c->num_batches * kMaxParts;
     k_hqs_tiled<BLOCK, TILE_PIX, PASS><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->d_levels, c->d_list, st, c->d_lo,
                                                                    c->d_med, c->d_hi, c->d_rgba, v, fb->d_depth,
-                                                                   fb->d_acc, occl ? 1 : 0, c->num_batches);
+                                                                   fb->d_acc, occl ? 1 : 0, c->num_batches, c->d_gbox,
+                                                                   c->d_gbase);
 }
 
 template <int BLOCK, int TILE_PIX>
@@ -1996,7 +2232,7 @@ int launch_hqs_tiled(hipStream_t s, const pcr_cloud* c, const pcr_view& v, int t
 // the batch, as k_mv_raster_tiled does for keys. Pass 1 takes items from
 // queue_head, pass 2 from queue_head2.
 template <int BLOCK, int TILE_PIX, int PASS>
-__global__ __launch_bounds__(BLOCK) void k_mv_hqs_tiled(const pcr_batch* __restrict__ b, uint32_t nb,
+__global__ __launch_bounds__(BLOCK, PASS == 1 && TILE_PIX <= 2048 ? 4 : 1) void k_mv_hqs_tiled(const pcr_batch* __restrict__ b, uint32_t nb,
                                                         const uint8_t* __restrict__ levels,
                                                         const uint32_t* __restrict__ list, MVState* __restrict__ st,
                                                         const uint32_t* __restrict__ lo,
@@ -2005,7 +2241,10 @@ __global__ __launch_bounds__(BLOCK) void k_mv_hqs_tiled(const pcr_batch* __restr
                                                         const uint32_t* __restrict__ rgba,
                                                         const pcr_view* __restrict__ views, int nviews,
                                                         uint32_t* const* __restrict__ depths,
-                                                        uint32_t* const* __restrict__ accs, int occl) {
+                                                        uint32_t* const* __restrict__ accs, int occl,
+                                                        const uint2* __restrict__ gbox,
+                                                        const uint32_t* __restrict__ gbase) {
+    __shared__ HqsGroups<BLOCK> hg;
     __shared__ HqsTile<PASS, TILE_PIX> tile;
     __shared__ uint32_t tile2[PASS == 0 ? TILE_PIX : 1];   // pass 1: the second view of a pair
     __shared__ uint32_t s_item, s_nv;
@@ -2057,7 +2296,8 @@ __global__ __launch_bounds__(BLOCK) void k_mv_hqs_tiled(const pcr_batch* __restr
                     if (lv == lj && hqs2_pair_batch<BLOCK, TILE_PIX, false>(bi, lv, b, lo, med, hi, rgba, views[vi],
                                                                              depths[vi], accs[vi], views[vj],
                                                                              depths[vj], accs[vj], tile.depth,
-                                                                             tile.acc, occl != 0, part, nparts)) {
+                                                                             tile.acc, occl != 0, part, nparts,
+                                                                             gbox ? gbox + gbase[bi] : nullptr, hg)) {
                         __syncthreads();   // the tile is reused by the next views
                         k += 2;
                         continue;
@@ -2065,7 +2305,9 @@ __global__ __launch_bounds__(BLOCK) void k_mv_hqs_tiled(const pcr_batch* __restr
                 }
             }
             hqs_tiled_batch<BLOCK, TILE_PIX, PASS, false>(bi, lv, b, lo, med, hi, rgba, views[vi], depths[vi],
-                                                           accs[vi], tile.depth, tile.acc, occl != 0, part, nparts);
+                                                           accs[vi], tile.depth, tile.acc, occl != 0, part, nparts,
+                                                           gbox ? gbox + gbase[bi] : nullptr,
+                                                           &hg);
             __syncthreads();   // the tile is reused by the next view
             k++;
         }
@@ -2090,7 +2332,7 @@ static void mv_hqs_tiled_t(hipStream_t s, const pcr_cloud* c, const MVBuffers& B
     k_mv_hqs_tiled<BLOCK, TILE_PIX, PASS><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->num_batches, B.d_levels,
                                                                       B.d_list, B.d_state, c->d_lo, c->d_med, c->d_hi,
                                                                       c->d_rgba, B.d_views, nviews, B.d_depths,
-                                                                      B.d_accs, occl ? 1 : 0);
+                                                                      B.d_accs, occl ? 1 : 0, c->d_gbox, c->d_gbase);
 }
 
 template <int BLOCK, int TILE_PIX>

@@ -139,3 +139,26 @@ def test_grouped_raster_equals_oracle(ctx, n, size, shift, shuffle, tile_px, blo
         assert np.array_equal(fb.keys(), ref) and ctx.stats().points_occluded == 0
         fb.close()
     cloud.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,size,shift,shuffle", [(1000, 63, True, False), (20011, 1025, True, False),
+                                                  (150_001, 10240, True, False), (150_001, 16385, True, True),
+                                                  (200_003, 200_003, True, False)])
+@pytest.mark.parametrize("tile_px,block", [(2048, 256), (1024, 128), (4096, 256)])
+def test_grouped_hqs_equals_the_direct_passes(ctx, n, size, shift, shuffle, tile_px, block):
+    """The direct passes (tile_px 0) are compared with the oracle elsewhere."""
+    b, lo, med, hi, rgba = layout(n, size, shift, shuffle)
+    cloud = ctx.upload_batched(b, lo, med, hi, rgba)
+    for v in views():
+        ref = ctx.framebuffer(v.width, v.height, pcr.FB_HQS)
+        ctx.render(cloud, v, pcr.params(pcr.MODE_HQS, tile_px=0), ref)
+        for skip in (True, False):
+            fb = ctx.framebuffer(v.width, v.height, pcr.FB_HQS)
+            ctx.render(cloud, v, pcr.params(pcr.MODE_HQS, tile_px=tile_px, block_size=block, occlusion_skip=skip), fb)
+            st = ctx.stats()
+            assert all(np.array_equal(a, r) for a, r in zip(fb.hqs(), ref.hqs()))
+            assert st.points_occluded <= 2 * st.points_drawn and (skip or st.points_occluded == 0)
+            fb.close()
+        ref.close()
+    cloud.close()

@@ -992,7 +992,7 @@ __device__ __forceinline__ BatchRun next_run(const uint2* __restrict__ box, uint
 // of the parts cost the overview a fifth wave per SIMD's worth of latency. A
 // kernel of its own for the large batches, before this one, was slower (443
 // us): its waits for memory no longer overlap the other batches' arithmetic.
-template <int BLOCK, int TILE_PIX>
+template <int BLOCK, int TILE_PIX, bool NT>
 __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const pcr_batch* __restrict__ b,
                                                   const uint32_t* __restrict__ lo, const uint32_t* __restrict__ med,
                                                   const uint32_t* __restrict__ hi, const pcr_view& v,
@@ -1049,11 +1049,11 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
             const Proj pj = make_proj(v.transform, v.width, v.height);
             if (use) {
                 if (seen == 2 && level >= 2 && interior) {
-                    tile_groups<BLOCK, true>(d, lo, parted ? box + (h.first_point - (h.first_point & 3u) - (first - lead)) / kGroupPoints : box,
+                    tile_groups<BLOCK, NT>(d, lo, parted ? box + (h.first_point - (h.first_point & 3u) - (first - lead)) / kGroupPoints : box,
                                              h, v, pj, group_slack(v.transform, h.min, h.max, v.width, v.height, wnear),
                                              fb, tile, x0, y0, tw, th, natom, gl);
                 } else {
-                    tile_dispatch<BLOCK, true, true>(level, d, lo, med, hi, h, pj, fb, tile, x0, y0, tw, th, natom,
+                    tile_dispatch<BLOCK, true, NT>(level, d, lo, med, hi, h, pj, fb, tile, x0, y0, tw, th, natom,
                                                      interior);
                 }
                 __syncthreads();
@@ -1061,7 +1061,7 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
                 tile_flush<BLOCK>(tile, fb, x0, y0, tw, n, magic, (uint32_t)v.width, natom, h.first_point,
                                   h.num_points);
             } else {
-                tile_dispatch<BLOCK, false, true>(level, d, lo, med, hi, h, pj, fb, nullptr, 0, 0, 0, 0, natom);
+                tile_dispatch<BLOCK, false, NT>(level, d, lo, med, hi, h, pj, fb, nullptr, 0, 0, 0, 0, natom);
             }
         }
         if (!parted || g >= ng) break;
@@ -1106,7 +1106,7 @@ __global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_raster_tile
         const int level = __builtin_amdgcn_readfirstlane(levels[bi]);
         uint32_t skipped;
         if constexpr (GROUPS)
-            skipped = grouped_batch<BLOCK, TILE_PIX>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0, part,
+            skipped = grouped_batch<BLOCK, TILE_PIX, true>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0, part,
                                                      nparts, gbox + gbase[bi], groups);
         else
             skipped = tiled_batch<BLOCK, TILE_PIX, true>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0,
@@ -1281,15 +1281,23 @@ __device__ __forceinline__ bool raster_pair_batch(uint32_t bi, int level, const 
     return true;
 }
 
+// With group bounds a view drawn by itself takes grouped_batch(): a large batch
+// in parts, hidden groups left out. Six waves per SIMD: without the bound the
+// kernel has 108 registers and four waves, and 48 views of a 1e9-point city
+// take 13.9 ms; with it 11.4, and 12.3 without the groups. The pairs stay: with
+// grouped_batch() for every view by itself the launch takes 11.8.
 template <int BLOCK, int TILE_PIX>
-__global__ __launch_bounds__(BLOCK) void k_mv_raster_tiled(const pcr_batch* __restrict__ b, uint32_t nb,
+__global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_mv_raster_tiled(const pcr_batch* __restrict__ b, uint32_t nb,
                                                            const uint8_t* __restrict__ levels,
                                                            const uint32_t* __restrict__ list,
                                                            MVState* __restrict__ st, const uint32_t* __restrict__ lo,
                                                            const uint32_t* __restrict__ med,
                                                            const uint32_t* __restrict__ hi,
                                                            const pcr_view* __restrict__ views, int nviews,
-                                                           unsigned long long* const* __restrict__ fbs, int occl) {
+                                                           unsigned long long* const* __restrict__ fbs, int occl,
+                                                           const uint2* __restrict__ gbox,
+                                                           const uint32_t* __restrict__ gbase) {
+    __shared__ GroupList<BLOCK> groups;
     __shared__ unsigned long long tile[TILE_PIX];
     __shared__ uint32_t s_item, s_nv;
     __shared__ uint8_t s_vid[64], s_lv[64];
@@ -1346,7 +1354,11 @@ __global__ __launch_bounds__(BLOCK) void k_mv_raster_tiled(const pcr_batch* __re
                     continue;
                 }
             }
-            tiled_batch<BLOCK, TILE_PIX, false, true>(bi, lv, b, lo, med, hi, views[vi], fbs[vi], tile, &s_natom,
+            if (gbox)
+                grouped_batch<BLOCK, TILE_PIX, false>(bi, lv, b, lo, med, hi, views[vi], fbs[vi], tile, &s_natom,
+                                                      occl != 0, part, nparts, gbox + gbase[bi], groups);
+            else
+                tiled_batch<BLOCK, TILE_PIX, false, true>(bi, lv, b, lo, med, hi, views[vi], fbs[vi], tile, &s_natom,
                                                       occl != 0, part, nparts, &ra);
             __syncthreads();   // the tile is reused by the next view
             k++;
@@ -1370,7 +1382,7 @@ static void mv_tiled_t(hipStream_t s, const pcr_cloud* c, const MVBuffers& B, in
     if (grid == 0) grid = 1;
     k_mv_raster_tiled<BLOCK, TILE_PIX><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->num_batches, B.d_levels, B.d_list,
                                                                   B.d_state, c->d_lo, c->d_med, c->d_hi, B.d_views,
-                                                                  nviews, B.d_fbs, occl ? 1 : 0);
+                                                                  nviews, B.d_fbs, occl ? 1 : 0, c->d_gbox, c->d_gbase);
 }
 
 int launch_mv_raster_tiled(hipStream_t s, const pcr_cloud* c, const MVBuffers& B, int nviews, int tile_px, int block,

@@ -117,9 +117,10 @@ typedef struct pcr_render_params {
     int32_t  time_stages;       /* 1: record HIP events around each stage; 2:
                                    around the raster stage only (two events a
                                    frame instead of six; see pcr_frame_times)    */
-    int32_t  tile_px;           /* LAS2/NODES/HQS/NODES_HQS: batches whose screen
-                                   rectangle fits in this many pixels merge in an
-                                   LDS tile first (0 = off, else 1024/2048/4096);
+    int32_t  tile_px;           /* LAS2/NODES/HQS/NODES_HQS: batches (or parts of
+                                   them) whose screen rectangle fits in this many
+                                   pixels merge in an LDS tile first (0 = off, else
+                                   1024/2048/4096);
                                    same result. For hqs it also merges the colour
                                    sums, which is what makes dense views fast    */
     uint32_t batch_begin;       /* draw batches [batch_begin, batch_end) only;     */
@@ -135,9 +136,10 @@ typedef struct pcr_render_params {
                                    148-191 carries switched off (its constant is
                                    0.0005); 0 = off                              */
     int32_t  occlusion_skip;    /* tiled LAS2/NODES/HQS/NODES_HQS raster: 0 = on
-                                   (default), -1 = off. A batch whose nearest
-                                   possible depth lies behind every depth already
-                                   drawn over its screen rectangle is skipped;
+                                   (default), -1 = off. A batch, or 64 points of
+                                   one, whose nearest possible depth lies behind
+                                   every depth already drawn over its screen
+                                   rectangle is skipped;
                                    the frame is the same bit for bit either way */
     int32_t  debug_counters;    /* 1: the index resolve also counts the covered
                                    pixels (pcr_stats.pixels_visible), as the

@@ -563,10 +563,12 @@ int pcr_stats_get(pcr_ctx* ctx, pcr_stats* out) {
     for (int i = 0; i < 5; i++) out->batches_per_level[i] = st.level_count[i];
     out->points_drawn = st.points_drawn;
     out->bytes_algorithmic = st.plane_bytes + 64ull * ctx->last_nb;
-    out->batches_occluded = st.occluded_batches;
-    out->points_occluded = st.occluded_points;
-    out->bytes_occluded = st.occluded_bytes;
-    out->atomics_issued = st.atomics;
+    for (const FrameCounts& c : st.counts) {
+        out->batches_occluded += c.occluded_batches;
+        out->points_occluded += c.occluded_points;
+        out->bytes_occluded += c.occluded_bytes;
+        out->atomics_issued += c.atomics;
+    }
     out->pixels_visible = st.pixels_visible;
     if (ctx->timing && ctx->frames_timed) {
         hipEvent_t* ev = ctx->ring[(ctx->frames_timed - 1) % PCR_TIMING_RING];

@@ -62,14 +62,19 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
 // ------------------------------------------------------------------ fills
 // A frame's counters are zeroed by the select launch of the frame before it
 // (k_select resets the other of the context's two frame states).
-__device__ __forceinline__ void frame_reset(FrameState* st) {
+__device__ __forceinline__ void frame_reset(FrameState* st, uint32_t thread) {
+    if (thread < kCountSlots) {
+        FrameCounts* c = st->counts + thread;
+        c->occluded_points = 0; c->occluded_bytes = 0; c->atomics = 0; c->occluded_batches = 0;
+    }
+    if (thread != 0) return;
     for (uint32_t k = 0; k < kSlices; k++) st->slice_count[k] = 0;
     st->queue_head = 0; st->queue_head2 = 0; st->culled = 0;
     for (int i = 0; i < 5; i++) st->level_count[i] = 0;
     st->points_drawn = 0; st->plane_bytes = 0;
-    st->occluded_batches = 0; st->occluded_points = 0; st->occluded_bytes = 0; st->atomics = 0;
     st->pixels_visible = 0;
 }
+__device__ __forceinline__ FrameCounts* frame_counts(FrameState* st) { return st->counts + blockIdx.x % kCountSlots; }
 // 16-byte stores (p is hipMalloc-aligned); the last element of an odd-length
 // 64-bit fill, or the last 1-3 of a 32-bit fill, are stored singly.
 __global__ void k_fill64(unsigned long long* __restrict__ p, uint64_t n, unsigned long long v) {
@@ -88,7 +93,7 @@ __global__ void k_fill32(uint32_t* __restrict__ p, uint64_t n, uint32_t v) {
     if (t < (n & 3)) p[(n & ~3ull) + t] = v;
 }
 __global__ void k_frame_reset(FrameState* st) {
-    if (threadIdx.x == 0) frame_reset(st);
+    frame_reset(st, threadIdx.x);
 }
 
 static int grid_for(uint64_t n, int block) {
@@ -159,7 +164,7 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(const pcr_batch* __rest
     {
         const uint64_t t = (uint64_t)blockIdx.x * kSelectBlock + threadIdx.x;
         const uint64_t stride = (uint64_t)gridDim.x * kSelectBlock;
-        if (t == 0) frame_reset(st_next);
+        if (blockIdx.x == 0) frame_reset(st_next, threadIdx.x);
         fill_words(fill0, t, stride);
         fill_words(fill1, t, stride);
     }
@@ -361,7 +366,7 @@ __global__ __launch_bounds__(BLOCK) void k_raster_batched(const pcr_batch* __res
         else raster_strided<BLOCK, 2>(d, lo, med, hi, h.first_point, h.num_points, v, fb, natom);
     }
     const unsigned long long wa = wave_sum_u64(natom);
-    if (__lane_id() == 0 && wa) atomicAdd(&st->atomics, wa);
+    if (__lane_id() == 0 && wa) atomicAdd(&frame_counts(st)->atomics, wa);
 }
 
 template <int BLOCK, int VEC>
@@ -1127,11 +1132,12 @@ __global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_raster_tile
         __syncthreads();   // s_item and the tile are reused by the next item
     }
     // the loop ends after a barrier that follows every thread's last atomic
-    if (threadIdx.x == 0 && s_natom) atomicAdd(&st->atomics, (unsigned long long)s_natom);
+    if (threadIdx.x == 0 && s_natom) atomicAdd(&frame_counts(st)->atomics, (unsigned long long)s_natom);
     if (threadIdx.x == 0 && s_occ_points) {
-        atomicAdd(&st->occluded_batches, s_occ_batches);
-        atomicAdd(&st->occluded_points, s_occ_points);
-        atomicAdd(&st->occluded_bytes, s_occ_bytes);
+        FrameCounts* c = frame_counts(st);
+        atomicAdd(&c->occluded_batches, s_occ_batches);
+        atomicAdd(&c->occluded_points, s_occ_points);
+        atomicAdd(&c->occluded_bytes, s_occ_bytes);
     }
 }
 
@@ -2266,9 +2272,10 @@ void k_hqs_tiled(const pcr_batch* __restrict__ b,
         __syncthreads();   // s_item and the tile are reused by the next item
     }
     if (threadIdx.x == 0 && s_occ_points) {
-        atomicAdd(&st->occluded_batches, s_occ_batches);
-        atomicAdd(&st->occluded_points, s_occ_points);
-        atomicAdd(&st->occluded_bytes, s_occ_bytes);
+        FrameCounts* c = frame_counts(st);
+        atomicAdd(&c->occluded_batches, s_occ_batches);
+        atomicAdd(&c->occluded_points, s_occ_points);
+        atomicAdd(&c->occluded_bytes, s_occ_bytes);
     }
 }
 

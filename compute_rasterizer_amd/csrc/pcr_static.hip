@@ -22,11 +22,10 @@
 namespace pcr {
 namespace {
 
-constexpr uint64_t kStateBytes = 256;                                      // two FrameStates
+constexpr uint64_t kStateBytes = 2 * sizeof(FrameState);
 constexpr uint64_t kListBytes = 4ull * PCR_STATIC_MAX_BATCHES;             // drawn-batch list
 constexpr uint64_t kLevelBytes = 1ull * PCR_STATIC_MAX_BATCHES;            // per-batch level
 constexpr uint64_t kScratchBytes = kStateBytes + kListBytes + kLevelBytes;
-static_assert(2 * sizeof(FrameState) <= kStateBytes, "frame states exceed their slot");
 static_assert(kStateBytes % 16 == 0 && kListBytes % 16 == 0, "list and levels keep 16-byte alignment");
 constexpr int kMaxDevices = 64;
 

@@ -9,6 +9,8 @@
 //   k_hqs_*           two-pass depth + accumulate (compute_loop_las_hqs/depth.cs, color.cs)
 //   k_resolve_*       to RGBA8 (compute_loop_las/resolve.cs:100-146, hqs/resolve.cs:62-129,
 //                     compute_2021_earlyz/resolve.cs:41-78)
+#include <algorithm>
+#include <cmath>
 #include "pcr_device.h"
 #include "pcr_internal.h"
 
@@ -1001,7 +1003,7 @@ __device__ __forceinline__ BatchRun next_run(const uint2* __restrict__ box, uint
 // of the parts cost the overview a fifth wave per SIMD's worth of latency. A
 // kernel of its own for the large batches, before this one, was slower (443
 // us): its waits for memory no longer overlap the other batches' arithmetic.
-template <int BLOCK, int TILE_PIX, bool NT>
+template <int BLOCK, int TILE_PIX, bool NT, bool PARTS>
 __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const pcr_batch* __restrict__ b,
                                                   const uint32_t* __restrict__ lo, const uint32_t* __restrict__ med,
                                                   const uint32_t* __restrict__ hi, const pcr_view& v,
@@ -1021,7 +1023,7 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
     bool use = screen_rect(v.transform, h.min, h.max, v.width, v.height, x0, y0, x1, y1, &interior, &wlo, &wnear);
     int tw = x1 - x0 + 1, th = y1 - y0 + 1;
     const auto fits = [](int w, int hh) { return run_fits<TILE_PIX>(w, hh); };
-    const bool parted = use && !fits(tw, th) && wnear > 0.0f;
+    const bool parted = PARTS && use && !fits(tw, th) && wnear > 0.0f;
     const uint32_t first = h.first_point, np = h.num_points, lead = first & 3u, ng = groups_of(first, np);
     uint32_t skipped = 0, g = 0;   // g: the first group not yet drawn
     for (;;) {
@@ -1081,13 +1083,22 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
 
 // Persistent workgroups take drawn batches from the select stage's compacted
 // list through an atomic queue, so no workgroup is launched for a culled
-// batch. The loop ends when the queue passes list_count, which every
+// batch. The loop ends when the queue passes the last work item, which every
 // workgroup reaches.
-// GROUPS: the cloud has group bounds. Six waves per SIMD: with eight the
-// batch state spills inside the loops (361 us for the frame above, 340 with
-// seven, 333 with six).
-template <int BLOCK, int TILE_PIX, bool GROUPS>
-__global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_raster_tiled(const pcr_batch* __restrict__ b,
+// kParts runs six waves per SIMD: with eight the batch state spills inside the
+// loops (a 1e9-point city from 100 m 361 us, 340 with seven, 333 with six, all
+// before the counters had lines of their own). Without the parts eight fit: a
+// 400M-point terrain from above takes 571 us, with parts 632, and as much with
+// every test off, so it is the waves that count there.
+enum RasterKind {
+    kNoGroups,   // no group bounds: tiled_batch()
+    kParts,      // grouped_batch(), a batch larger than the tile in parts
+    kWhole       // grouped_batch(), a batch larger than the tile point by point (far_view)
+};
+// The tile leaves LDS for more than six waves per SIMD.
+constexpr bool waves_bound(int block, int tile_px) { return tile_px <= 8 * block; }
+template <int BLOCK, int TILE_PIX, int KIND>
+__global__ __launch_bounds__(BLOCK, !waves_bound(BLOCK, TILE_PIX) ? 1 : KIND == kParts ? 6 : 8) void k_raster_tiled(const pcr_batch* __restrict__ b,
                                                         const uint8_t* __restrict__ levels,
                                                         const uint32_t* __restrict__ list,
                                                         FrameState* __restrict__ st,
@@ -1114,8 +1125,8 @@ __global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_raster_tile
         const uint32_t bi = __builtin_amdgcn_readfirstlane(list[slot]);
         const int level = __builtin_amdgcn_readfirstlane(levels[bi]);
         uint32_t skipped;
-        if constexpr (GROUPS)
-            skipped = grouped_batch<BLOCK, TILE_PIX, true>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0, part,
+        if constexpr (KIND != kNoGroups)
+            skipped = grouped_batch<BLOCK, TILE_PIX, true, KIND == kParts>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0, part,
                                                      nparts, gbox + gbase[bi], groups);
         else
             skipped = tiled_batch<BLOCK, TILE_PIX, true>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0,
@@ -1141,12 +1152,12 @@ __global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_raster_tile
     }
 }
 
-template <int BLOCK, int TILE_PIX, bool GROUPS>
+template <int BLOCK, int TILE_PIX, int KIND>
 static void tiled_grid(hipStream_t s, const pcr_cloud* c, const pcr_view& v, FrameState* st, unsigned long long* fb,
                     bool occl) {
     static const int occ = [] {
         int o = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, k_raster_tiled<BLOCK, TILE_PIX, GROUPS>, BLOCK, 0) != hipSuccess) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, k_raster_tiled<BLOCK, TILE_PIX, KIND>, BLOCK, 0) != hipSuccess) {
             (void)hipGetLastError();
             o = 0;
         }
@@ -1154,16 +1165,50 @@ static void tiled_grid(hipStream_t s, const pcr_cloud* c, const pcr_view& v, Fra
     }();
     uint64_t grid = (uint64_t)c->ctx->cu_count * (uint64_t)occ;
     if (grid > (uint64_t)c->num_batches * kMaxParts) grid = (uint64_t)c->num_batches * kMaxParts;
-    k_raster_tiled<BLOCK, TILE_PIX, GROUPS><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->d_levels, c->d_list, st, c->d_lo,
+    k_raster_tiled<BLOCK, TILE_PIX, KIND><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->d_levels, c->d_list, st, c->d_lo,
                                                                c->d_med, c->d_hi, v, fb, occl ? 1 : 0,
                                                                c->num_batches, c->d_gbox, c->d_gbase);
+}
+
+// Whether k_raster_tiled draws the view's batches whole (kWhole): the cloud's
+// box lies in front of the eye as a whole, and a batch of the median size,
+// seen at the distance of the box's centre, measures at most 11 pixels.
+// Few batches are then larger than the tile, and the frame gains more from
+// eight waves per SIMD than from the parts. Measured whole and in parts, from
+// above and from outside (us): 400M points at 7.4 px 571 and 632 (terrain), at
+// 6.5 px 473 and 517 (city); 200M at 10.4 px 325 and 350 (terrain), at 10.9 px
+// 266 and 269, at 12.1 px 402 and 341, and 100M at 12.8 px 240 and 201 (city).
+// The line follows the tile's side (1024 pixels, 200M points at 9.0 px: 399 and
+// 320). The nodes of an octree differ too much in size for a median to tell.
+static bool far_view(const pcr_cloud* c, const pcr_view& v, int tile_px) {
+    const double far_px = 11.0 * std::sqrt(tile_px / 2048.0);   // of a 2048-pixel tile: 11
+    const float* t = v.transform;
+    if (!(c->batch_edge > 0.0f) || c->num_levels > 0) return false;
+    double nearest = t[15], centre = t[15], x = 0, y = 0;
+    for (int a = 0; a < 3; a++) {
+        const double tw = t[4 * a + 3], lo = tw * c->aabb_min[a], hi = tw * c->aabb_max[a];
+        nearest += lo < hi ? lo : hi;
+        centre += 0.5 * (lo + hi);
+        x += (double)t[4 * a] * t[4 * a];
+        y += (double)t[4 * a + 1] * t[4 * a + 1];
+    }
+    const double px = 0.5 * std::max(v.width * std::sqrt(x), v.height * std::sqrt(y)) * c->batch_edge;
+    return nearest > 0 && px <= far_px * centre;
 }
 
 template <int BLOCK, int TILE_PIX>
 static void tiled_t(hipStream_t s, const pcr_cloud* c, const pcr_view& v, FrameState* st, unsigned long long* fb,
                     bool occl) {
-    if (c->d_gbox) tiled_grid<BLOCK, TILE_PIX, true>(s, c, v, st, fb, occl);
-    else tiled_grid<BLOCK, TILE_PIX, false>(s, c, v, st, fb, occl);
+    if (!c->d_gbox) {
+        tiled_grid<BLOCK, TILE_PIX, kNoGroups>(s, c, v, st, fb, occl);
+        return;
+    }
+    if constexpr (waves_bound(BLOCK, TILE_PIX))
+        if (far_view(c, v, TILE_PIX)) {
+            tiled_grid<BLOCK, TILE_PIX, kWhole>(s, c, v, st, fb, occl);
+            return;
+        }
+    tiled_grid<BLOCK, TILE_PIX, kParts>(s, c, v, st, fb, occl);
 }
 
 int launch_raster_tiled(hipStream_t s, const pcr_cloud* c, const pcr_view& v, int tile_px, int block,
@@ -1436,7 +1481,7 @@ __global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_mv_raster_t
                 }
             }
             if (gbox)
-                grouped_batch<BLOCK, TILE_PIX, false>(bi, lv, b, lo, med, hi, views[vi], fbs[vi], tile, &s_natom,
+                grouped_batch<BLOCK, TILE_PIX, false, true>(bi, lv, b, lo, med, hi, views[vi], fbs[vi], tile, &s_natom,
                                                       occl != 0, part, nparts, gbox + gbase[bi], groups[0]);
             else
                 tiled_batch<BLOCK, TILE_PIX, false, true>(bi, lv, b, lo, med, hi, views[vi], fbs[vi], tile, &s_natom,

@@ -319,6 +319,7 @@ int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
     const uint32_t nb = c->num_batches;
     if (nb == 0) return PCR_OK;
     std::vector<uint32_t> base(nb);
+    std::vector<float> edge(nb);
     uint64_t total = 0;
     uint32_t longest = 0;
     for (uint32_t i = 0; i < nb; i++) {
@@ -326,6 +327,9 @@ int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
         const uint32_t ng = groups_of(c->h_batches[i].first_point, c->h_batches[i].num_points);
         total += ng;
         longest = ng > longest ? ng : longest;
+        float e[3];   // two longest edges: the face a batch shows
+        for (int a = 0; a < 3; a++) e[a] = std::max(0.0f, c->h_batches[i].max[a] - c->h_batches[i].min[a]);
+        edge[i] = std::sqrt(std::max(e[0] * e[1], e[2] * std::max(e[0], e[1])));
     }
     if (total == 0 || total >= (1ull << 32)) return PCR_OK;
     uint2* box = nullptr;
@@ -342,6 +346,8 @@ int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
     PCR_HIP(hipGetLastError());
     PCR_HIP(hipStreamSynchronize(s));
     c->device_bytes += total * sizeof(uint2) + nb * sizeof(uint32_t);
+    std::nth_element(edge.begin(), edge.begin() + nb / 2, edge.end());
+    c->batch_edge = edge[nb / 2];
     return PCR_OK;
 }
 

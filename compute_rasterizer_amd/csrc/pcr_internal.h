@@ -15,6 +15,54 @@ __host__ __device__ inline uint32_t groups_of(uint32_t first, uint32_t n) {
     return (uint32_t)(((uint64_t)n + (first & 3u) + kGroupPoints - 1) / kGroupPoints);
 }
 
+// How the persistent workgroups of a launch share out its listed batches: the
+// last nsplit batches (one per workgroup) in nparts parts each, so that the
+// workgroups end together, and all of a list of fewer batches than half the
+// workgroups in as many parts as give each workgroup one.
+constexpr uint32_t kMaxParts = 16;
+struct ItemSplit {
+    uint32_t whole, nsplit, nparts, items;
+    __host__ __device__ inline void split(uint32_t count, uint32_t groups) {
+        nsplit = count < groups ? count : groups;
+        whole = count - nsplit;
+        nparts = 2u;
+        if (count && count * 2u <= groups) nparts = groups / count < kMaxParts ? groups / count : kMaxParts;
+        items = whole + nsplit * nparts;
+    }
+    // place in the list, part and number of parts of an item; first come the
+    // first parts of all split batches, then the second ones, and so on
+    __host__ __device__ inline uint32_t batch_of(uint32_t item, uint32_t& part, uint32_t& parts) const {
+        part = 0;
+        parts = 1;
+        if (item < whole) return item;
+        const uint32_t h = item - whole;
+        part = h / nsplit;
+        parts = nparts;
+        return whole + (h - part * nsplit);
+    }
+};
+// The points of one part of a batch: whole groups of 1024 points, one round of
+// a 256-thread workgroup (counted from the aligned word that the point loops
+// start at), so that no part ends in a round with idle threads. A part past
+// the last group is empty.
+constexpr uint32_t kPartRound = 1024;
+__host__ __device__ inline uint64_t part_words(uint32_t lead, uint32_t np, uint32_t nparts) {
+    const uint32_t rounds = (uint32_t)(((uint64_t)np + lead + kPartRound - 1) / kPartRound);
+    return (uint64_t)((rounds + nparts - 1) / nparts) * kPartRound;
+}
+__host__ __device__ inline bool part_empty(uint32_t first, uint32_t np, uint32_t part, uint32_t nparts) {
+    const uint32_t lead = first & 3u;
+    return np == 0 || part_words(lead, np, nparts) * part >= (uint64_t)np + lead;
+}
+__host__ __device__ inline void batch_part(pcr_batch& h, uint32_t part, uint32_t nparts) {
+    const uint32_t lead = h.first_point & 3u;
+    const uint64_t k = part_words(lead, h.num_points, nparts);
+    const uint64_t w0 = k * part, end = (uint64_t)h.num_points + lead;
+    const uint64_t lo = w0 > lead ? w0 - lead : 0, hi = w0 + k < end ? w0 + k - lead : h.num_points;
+    h.first_point += (uint32_t)(lo < h.num_points ? lo : h.num_points);
+    h.num_points = lo < hi ? (uint32_t)(hi - lo) : 0u;
+}
+
 // The select stage lists the drawn batches in kSlices slices of the view
 // depth, the nearest first: slice k of a cloud of nb batches starts at
 // list[k * nb].

@@ -609,8 +609,8 @@ __device__ __forceinline__ RectInfo uniform_rect(const RectInfo& s) {
     return r;
 }
 
-// The order in which a launch's persistent workgroups draw `count` listed
-// batches, as work items of whole batches or of parts of one.
+// The order in which a launch's persistent workgroups draw the listed batches,
+// as work items of whole batches or of parts of one (ItemSplit).
 //
 // The last nsplit batches (one per workgroup) are drawn in parts: workgroups
 // otherwise idle 43 us on average between their last batch and the end of
@@ -634,9 +634,7 @@ __device__ __forceinline__ RectInfo uniform_rect(const RectInfo& s) {
 //
 // The slices of the list (SliceRule) are drawn one after the other, the
 // nearest first; the spread is within a slice.
-constexpr uint32_t kMaxParts = 16;
-struct WorkItems {
-    uint32_t count, whole, nsplit, nparts, items;
+struct WorkItems : ItemSplit {
     // `start` (LDS, kSlices + 1 words) takes the first item of each slice;
     // every thread of the workgroup constructs it (it ends in a barrier)
     __device__ __forceinline__ WorkItems(const FrameState* st, uint32_t* start) {
@@ -649,43 +647,18 @@ struct WorkItems {
             start[kSlices] = n;
         }
         __syncthreads();
-        count = __builtin_amdgcn_readfirstlane(start[kSlices]);
-        nsplit = min(count, gridDim.x);
-        whole = count - nsplit;
-        nparts = count * 2u <= gridDim.x && count ? min(kMaxParts, gridDim.x / count) : 2u;
-        items = whole + nsplit * nparts;
+        split(__builtin_amdgcn_readfirstlane(start[kSlices]), gridDim.x);
     }
     // place in a list of nb entries a slice, part and number of parts of an item
     __device__ __forceinline__ uint64_t slot(uint32_t item, const uint32_t* start, uint32_t nb, uint32_t& part,
                                              uint32_t& parts) const {
-        part = 0;
-        parts = 1;
-        if (item >= whole) {
-            const uint32_t h = item - whole;
-            part = h / nsplit;
-            parts = nparts;
-            item = whole + (h - part * nsplit);
-        }
+        item = batch_of(item, part, parts);
         const unsigned long long m = __ballot(item >= start[__lane_id() & (kSlices - 1)]) & ((1ull << kSlices) - 1);
         const uint32_t k = (uint32_t)__popcll(m) - 1u;   // empty slices start where the next one does
         const uint32_t s0 = __builtin_amdgcn_readfirstlane(start[k]), n = __builtin_amdgcn_readfirstlane(start[k + 1]) - s0;
         return (uint64_t)k * nb + (uint32_t)(((uint64_t)(item - s0) * 2654435761ull) % n);
     }
 };
-// The points of one part of a batch: whole groups of 1024 points, one round of
-// a 256-thread workgroup (counted from the aligned word that the point loops
-// start at), so that no part ends in a round with idle threads. A part past
-// the last group is empty.
-__device__ __forceinline__ void batch_part(pcr_batch& h, uint32_t part, uint32_t nparts) {
-    constexpr uint32_t kRound = 1024;
-    const uint32_t lead = h.first_point & 3u, rounds = (uint32_t)(((uint64_t)h.num_points + lead + kRound - 1) / kRound);
-    const uint64_t k = (uint64_t)((rounds + nparts - 1) / nparts) * kRound;   // words per part
-    const uint64_t w0 = k * part, end = (uint64_t)h.num_points + lead;
-    const uint64_t lo = w0 > lead ? w0 - lead : 0, hi = w0 + k < end ? w0 + k - lead : h.num_points;
-    h.first_point += (uint32_t)(lo < h.num_points ? lo : h.num_points);
-    h.num_points = lo < hi ? (uint32_t)(hi - lo) : 0u;
-}
-
 // A persistent workgroup's next work item. The first is its own block index;
 // the others come from the launch's queue counter. Every workgroup increments
 // the one counter, and the memory performs atomics on one address one after
@@ -696,6 +669,10 @@ __device__ __forceinline__ void batch_part(pcr_batch& h, uint32_t part, uint32_t
 // every item to a workgroup of its own takes none. take() is called by every
 // thread of the workgroup; the returned item is workgroup-uniform. `s_item`
 // must not be rewritten before the workgroup's next barrier.
+// N: items per atomic. The items of a multi-view launch are many views long,
+// so there a second item in hand lengthens the end of the launch (50M points,
+// 8 views: 469 us, one at a time 429).
+template <uint32_t N = 2>
 struct QueueTake {
     uint32_t next;                 // the next item that is the workgroup's already, or none
     __device__ __forceinline__ QueueTake() : next(blockIdx.x) {}
@@ -706,10 +683,10 @@ struct QueueTake {
             return it;
         }
         if (items <= gridDim.x) return items;
-        if (threadIdx.x == 0) s_item = atomicAdd(head, 2u);
+        if (threadIdx.x == 0) s_item = atomicAdd(head, N);
         __syncthreads();
         const uint32_t it = gridDim.x + __builtin_amdgcn_readfirstlane(s_item);
-        next = it + 1u;
+        if (N == 2) next = it + 1u;
         return it;
     }
 };
@@ -1116,7 +1093,7 @@ __global__ __launch_bounds__(BLOCK, !waves_bound(BLOCK, TILE_PIX) ? 1 : KIND == 
     const WorkItems work(st, s_start);
     if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; s_natom = 0; }
     __syncthreads();
-    QueueTake q;
+    QueueTake<> q;
     for (;;) {
         const uint32_t item = q.take(&st->queue_head, s_item, work.items);
         if (item >= work.items) break;
@@ -1406,6 +1383,11 @@ __device__ __forceinline__ bool raster_pair_batch(uint32_t bi, int level, const 
     return true;
 }
 
+// The work items are those of k_raster_tiled without the slices. A short list
+// is split as there: in two parts a batch, 98 batches drawn for 30 views
+// took 810 us (as few workgroups, each all views one after the other), and
+// 485 in up to 16; 30 batches for two views 97 and 51.
+//
 // With group bounds a view drawn by itself takes grouped_batch(): a large batch
 // in parts, hidden groups left out. Six waves per SIMD: without the bound the
 // kernel has 108 registers and four waves, and 48 views of a 1e9-point city
@@ -1427,18 +1409,19 @@ __global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_mv_raster_t
     __shared__ uint32_t s_item, s_nv;
     __shared__ uint8_t s_vid[64], s_lv[64];
     __shared__ RectInfo s_rect[64];   // the batch's rectangle in each view that draws it
-    const uint32_t count = st->list_count;
-    const uint32_t nsplit = min(count, gridDim.x), whole = count - nsplit;
+    ItemSplit work;
+    work.split(st->list_count, gridDim.x);
     __shared__ uint32_t s_natom;   // counted, not reported per view
+    QueueTake<1> q;
     for (;;) {
-        if (threadIdx.x == 0) s_item = atomicAdd(&st->queue_head, 1u);
-        __syncthreads();
-        uint32_t item = __builtin_amdgcn_readfirstlane(s_item);
-        if (item >= count + nsplit) break;
-        // as in k_raster_tiled, the last item per workgroup is drawn as two halves
-        uint32_t part = 0, nparts = 1;
-        if (item >= whole) { part = (item - whole) & 1u; nparts = 2; item = whole + ((item - whole) >> 1); }
-        const uint32_t bi = __builtin_amdgcn_readfirstlane(list[item]);
+        const uint32_t item = q.take(&st->queue_head, s_item, work.items);
+        if (item >= work.items) break;
+        uint32_t part, nparts;
+        const uint32_t bi = __builtin_amdgcn_readfirstlane(list[work.batch_of(item, part, nparts)]);
+        if (nparts > 1 && part_empty(b[bi].first_point, b[bi].num_points, part, nparts)) {
+            __syncthreads();   // s_item is rewritten
+            continue;
+        }
         if (threadIdx.x < 64) {   // compact the views drawing this batch (wave 0)
             const int v = (int)threadIdx.x;
             const int lv = v < nviews ? levels[(uint64_t)v * nb + bi] : kCulled;
@@ -1504,7 +1487,7 @@ static void mv_tiled_t(hipStream_t s, const pcr_cloud* c, const MVBuffers& B, in
         return o > 0 ? o : 4;
     }();
     uint64_t grid = (uint64_t)cu_count * (uint64_t)occ;
-    if (grid > c->num_batches) grid = c->num_batches;
+    if (grid > (uint64_t)c->num_batches * kMaxParts) grid = (uint64_t)c->num_batches * kMaxParts;
     if (grid == 0) grid = 1;
     k_mv_raster_tiled<BLOCK, TILE_PIX><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->num_batches, B.d_levels, B.d_list,
                                                                   B.d_state, c->d_lo, c->d_med, c->d_hi, B.d_views,
@@ -2292,7 +2275,7 @@ void k_hqs_tiled(const pcr_batch* __restrict__ b,
     __shared__ unsigned long long s_occ_points, s_occ_bytes;   // what the occlusion test skipped
     if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; }
     __syncthreads();
-    QueueTake q;
+    QueueTake<> q;
     for (;;) {
         const uint32_t item = q.take(head, s_item, work.items);
         if (item >= work.items) break;
@@ -2389,17 +2372,18 @@ __global__ __launch_bounds__(BLOCK, PASS == 1 && TILE_PIX <= 2048 ? 4 : 1) void 
     __shared__ uint32_t s_item, s_nv;
     __shared__ uint8_t s_vid[64], s_lv[64];
     uint32_t* head = PASS == 0 ? &st->queue_head : &st->queue_head2;
-    const uint32_t count = st->list_count;
-    const uint32_t nsplit = min(count, gridDim.x), whole = count - nsplit;
+    ItemSplit work;
+    work.split(st->list_count, gridDim.x);
+    QueueTake<1> q;
     for (;;) {
-        if (threadIdx.x == 0) s_item = atomicAdd(head, 1u);
-        __syncthreads();
-        uint32_t item = __builtin_amdgcn_readfirstlane(s_item);
-        if (item >= count + nsplit) break;
-        // as in k_hqs_tiled, the last item per workgroup is drawn as two halves
-        uint32_t part = 0, nparts = 1;
-        if (item >= whole) { part = (item - whole) & 1u; nparts = 2; item = whole + ((item - whole) >> 1); }
-        const uint32_t bi = __builtin_amdgcn_readfirstlane(list[item]);
+        const uint32_t item = q.take(head, s_item, work.items);
+        if (item >= work.items) break;
+        uint32_t part, nparts;
+        const uint32_t bi = __builtin_amdgcn_readfirstlane(list[work.batch_of(item, part, nparts)]);
+        if (nparts > 1 && part_empty(b[bi].first_point, b[bi].num_points, part, nparts)) {
+            __syncthreads();   // s_item is rewritten
+            continue;
+        }
         if (threadIdx.x < 64) {   // compact the views drawing this batch (wave 0)
             const int v = (int)threadIdx.x;
             const int lv = v < nviews ? levels[(uint64_t)v * nb + bi] : kCulled;
@@ -2466,7 +2450,7 @@ static void mv_hqs_tiled_t(hipStream_t s, const pcr_cloud* c, const MVBuffers& B
         return o > 0 ? o : 4;
     }();
     uint64_t grid = (uint64_t)cu_count * (uint64_t)occ;
-    if (grid > c->num_batches) grid = c->num_batches;
+    if (grid > (uint64_t)c->num_batches * kMaxParts) grid = (uint64_t)c->num_batches * kMaxParts;
     if (grid == 0) grid = 1;
     k_mv_hqs_tiled<BLOCK, TILE_PIX, PASS><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->num_batches, B.d_levels,
                                                                       B.d_list, B.d_state, c->d_lo, c->d_med, c->d_hi,

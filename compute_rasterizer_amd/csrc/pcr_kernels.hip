@@ -622,9 +622,9 @@ __device__ __forceinline__ RectInfo uniform_rect(const RectInfo& s) {
 // first parts of all of them, then the second ones, and so on, so that a
 // pair of queue items never holds two parts of one batch. The raster of 10
 // batches of 10,240 points takes 8.5 us so, and 42 in two parts each; the hqs
-// passes over 350 octree nodes 78 + 116 us, and 184 + 140. From half the
-// workgroups on, two parts are as good as more (1,821 nodes: 228 us, 252 with
-// the old order of the parts).
+// passes over 350 octree nodes 78 + 116 us, and 184 + 140. Of a list longer
+// than the workgroups are many, two parts are as good as more (1,821 nodes:
+// 228 us, 252 with the old order of the parts).
 //
 // Consecutive items map to list slots spread over the whole list
 // (multiplying by a prime above any count, modulo the count, permutes the

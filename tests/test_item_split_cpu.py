@@ -71,3 +71,35 @@ def test_items_and_parts(tmp_path):
                     os.path.join(ROOT, "compute_rasterizer_amd", "csrc"), str(src), "-o", str(exe)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout
+
+
+ROUNDS = r"""
+#include <cstdio>
+#include "pcr_internal.h"
+using namespace pcr;
+int main() {
+    // between half the workgroups and all of them: halves of 977 batches on
+    // 1,536 workgroups end after a whole batch's time, thirds after two thirds
+    for (uint32_t groups : {1024u, 1536u, 2048u})
+        for (uint32_t count = groups / 2 + 1; count < groups; count++) {
+            ItemSplit w;
+            w.split(count, groups);
+            for (uint32_t p = 2; p <= 4; p++) {
+                const uint32_t mine = (count * w.nparts + groups - 1) / groups, other = (count * p + groups - 1) / groups;
+                if ((uint64_t)mine * p > (uint64_t)other * w.nparts) {
+                    std::printf("%u batches, %u workgroups: %u parts, %u better\n", count, groups, w.nparts, p);
+                    return 1;
+                }
+            }
+        }
+}
+"""
+
+
+def test_lists_near_the_number_of_workgroups(tmp_path):
+    src, exe = tmp_path / "rounds.cpp", tmp_path / "rounds"
+    src.write_text(ROUNDS)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I",
+                    os.path.join(ROOT, "compute_rasterizer_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout

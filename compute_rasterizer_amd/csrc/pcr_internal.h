@@ -170,6 +170,7 @@ struct pcr_cloud {
     uint32_t list_slices = 1;             // 1 or kSlices
     uint2* d_gbox = nullptr;              // coarse-plane bounds of each batch's groups (null: none)
     uint32_t* d_gbase = nullptr;          // per batch: its first group in d_gbox
+    bool unsorted = false;                // 64 consecutive points spread over most of their batch
     float batch_edge = 0;                 // median over the batches: root of the largest face (0: no group bounds)
     int num_levels = 0;                   // octree depth + 1 (LOD clouds)
     float aabb_min[3] = {0, 0, 0};

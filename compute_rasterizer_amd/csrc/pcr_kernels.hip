@@ -1070,7 +1070,7 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
 enum RasterKind {
     kNoGroups,   // no group bounds: tiled_batch()
     kParts,      // grouped_batch(), a batch larger than the tile in parts
-    kWhole       // grouped_batch(), a batch larger than the tile point by point (far_view)
+    kWhole       // grouped_batch(), a batch larger than the tile point by point (whole_batches)
 };
 // The tile leaves LDS for more than six waves per SIMD.
 constexpr bool waves_bound(int block, int tile_px) { return tile_px <= 8 * block; }
@@ -1157,10 +1157,14 @@ static void tiled_grid(hipStream_t s, const pcr_cloud* c, const pcr_view& v, Fra
 // 266 and 269, at 12.1 px 402 and 341, and 100M at 12.8 px 240 and 201 (city).
 // The line follows the tile's side (1024 pixels, 200M points at 9.0 px: 399 and
 // 320). The nodes of an octree differ too much in size for a median to tell.
-static bool far_view(const pcr_cloud* c, const pcr_view& v, int tile_px) {
+// A cloud in a random order of points has no parts smaller than its batches,
+// and is drawn whole too (10M points, from 100 m and from above: 125 and 276
+// us, in parts 151 and 315).
+static bool whole_batches(const pcr_cloud* c, const pcr_view& v, int tile_px) {
     const double far_px = 11.0 * std::sqrt(tile_px / 2048.0);   // of a 2048-pixel tile: 11
     const float* t = v.transform;
     if (!(c->batch_edge > 0.0f) || c->num_levels > 0) return false;
+    if (c->unsorted) return true;
     double nearest = t[15], centre = t[15], x = 0, y = 0;
     for (int a = 0; a < 3; a++) {
         const double tw = t[4 * a + 3], lo = tw * c->aabb_min[a], hi = tw * c->aabb_max[a];
@@ -1181,7 +1185,7 @@ static void tiled_t(hipStream_t s, const pcr_cloud* c, const pcr_view& v, FrameS
         return;
     }
     if constexpr (waves_bound(BLOCK, TILE_PIX))
-        if (far_view(c, v, TILE_PIX)) {
+        if (whole_batches(c, v, TILE_PIX)) {
             tiled_grid<BLOCK, TILE_PIX, kWhole>(s, c, v, st, fb, occl);
             return;
         }

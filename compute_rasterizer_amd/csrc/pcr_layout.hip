@@ -344,8 +344,31 @@ int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
     PCR_HIP(hipMemcpyAsync(c->d_gbase, base.data(), nb * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     k_group_box<<<dim3(nb, rows), 256, 0, s>>>(c->d_batches, c->d_gbase, c->d_lo, c->d_gbox);
     PCR_HIP(hipGetLastError());
+    // a sample of the groups: kRows runs of up to kRow, over the whole cloud
+    constexpr uint64_t kRows = 16, kRow = 256;
+    const uint64_t rows_n = total < kRows * kRow ? 1 : kRows, row = total < kRows * kRow ? total : kRow;
+    std::vector<uint2> sample(rows_n * row);
+    PCR_HIP(hipMemcpy2DAsync(sample.data(), row * sizeof(uint2), c->d_gbox, total / rows_n * sizeof(uint2),
+                             row * sizeof(uint2), rows_n, hipMemcpyDeviceToHost, s));
     PCR_HIP(hipStreamSynchronize(s));
     c->device_bytes += total * sizeof(uint2) + nb * sizeof(uint32_t);
+    double spread = 0;
+    for (uint64_t k = 0; k < sample.size(); k++) {
+        const uint32_t g = (uint32_t)(k / row * (total / rows_n) + k % row);
+        const pcr_batch& h = c->h_batches[std::upper_bound(base.begin(), base.end(), g) - base.begin() - 1];
+        float whole = 0, part = 0;
+        for (int a = 0; a < 3; a++) {
+            const float e = h.max[a] - h.min[a];
+            const int n = (int)((sample[k].y >> (10 * a)) & 1023u) - (int)((sample[k].x >> (10 * a)) & 1023u);
+            whole = std::max(whole, e);
+            part = std::max(part, e * (float)std::max(n, 0) / 1024.0f);
+        }
+        spread += whole > 0.0f ? part / whole : 0.0;
+    }
+    // 0.98 for points in a random order, 0.03 to 0.17 for sorted ones and for
+    // flight lines; 0.57 and 0.75 (a city, each building's points together)
+    // still gain from the parts
+    c->unsorted = spread > 0.8 * (double)sample.size();
     std::nth_element(edge.begin(), edge.begin() + nb / 2, edge.end());
     c->batch_edge = edge[nb / 2];
     return PCR_OK;

@@ -47,3 +47,33 @@ def test_far_views_equal_oracle(ctx, tile_px, block, dist):
         assert np.array_equal(fb.keys(), ref)
         fb.close()
     cloud.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,size", [(3000, 7), (70_003, 1024), (200_003, 10240)])
+def test_unsorted_points_equal_oracle(ctx, n, size):
+    """Points in a random order: every batch covers the scene, near and far."""
+    xyz, rgba = orc.generate(pcr.gen_cfg(pcr.SCENE_TERRAIN, n, seed=5))
+    perm = np.random.default_rng(6).permutation(n)
+    b, lo, med, hi = pcr.encode_batches_host(xyz[perm], (size + 3) // 4 * 4)
+    cloud = ctx.upload_batched(b, lo, med, hi, rgba[perm])
+    mid = 0.5 * (b["min"].min(0) + b["max"].max(0))
+    ext = float((b["max"].max(0) - b["min"].min(0)).max())
+    for dist in (0.0, 0.8, 20.0):   # inside, nearby, far
+        eye = mid + np.array([0.3, -0.2, 0.1]) * ext * (0.3 + 2 * dist)
+        v = pcr.look_at(tuple(map(float, eye)), tuple(map(float, mid)), up=(0, 0, 1), near=0.1, far=1e6, width=643, height=397)
+        ref, _ = orc.render_batched(b, lo, med, hi, v, 1)
+        direct = ctx.framebuffer(v.width, v.height, pcr.FB_HQS)
+        ctx.render(cloud, v, pcr.params(pcr.MODE_HQS, tile_px=0), direct)
+        for mode in (pcr.MODE_LAS2, pcr.MODE_LAS):
+            fb = ctx.framebuffer(v.width, v.height)
+            for clear in (True, False):
+                ctx.render(cloud, v, pcr.params(mode, clear_before=clear), fb)
+                assert np.array_equal(fb.keys(), ref)
+            fb.close()
+        hq = ctx.framebuffer(v.width, v.height, pcr.FB_HQS)
+        ctx.render(cloud, v, pcr.params(pcr.MODE_HQS), hq)
+        assert all(np.array_equal(a, r) for a, r in zip(hq.hqs(), direct.hqs()))
+        hq.close()
+        direct.close()
+    cloud.close()

@@ -279,12 +279,15 @@ int cloud_alloc_batched(pcr_ctx* ctx, uint32_t nb, uint64_t npoints, pcr_cloud* 
 }
 
 // Coarse-plane bounds of every group of kGroupPoints points: a 16-lane row of
-// a wave holds one group, a quad of words per lane. blockIdx.x is the batch;
-// the groups of long batches are spread over blockIdx.y. Packed as the plane's
-// words are: min in x, max in y. Bound by the one read of the coarse plane.
-__global__ __launch_bounds__(256) void k_group_box(const pcr_batch* __restrict__ b, const uint32_t* __restrict__ gbase,
-                                                   const uint32_t* __restrict__ lo, uint2* __restrict__ box) {
-    const uint32_t first = b[blockIdx.x].first_point, np = b[blockIdx.x].num_points;
+// a wave holds one group, a quad of words per lane. The workgroups of a row
+// take every gridDim.x-th batch (a grid has fewer than 2^32 threads, so not
+// one workgroup for each of 2^24 batches); the groups of long batches are
+// spread over blockIdx.y. Packed as the plane's words are: min in x, max in y.
+// Bound by the one read of the coarse plane.
+__device__ __forceinline__ void group_box(uint32_t bi, const pcr_batch* __restrict__ b,
+                                          const uint32_t* __restrict__ gbase, const uint32_t* __restrict__ lo,
+                                          uint2* __restrict__ box) {
+    const uint32_t first = b[bi].first_point, np = b[bi].num_points;
     const uint32_t lead = first & 3u, ng = groups_of(first, np), nq = (uint32_t)(((uint64_t)np + lead + 3u) >> 2);
     const u32x4* lo4 = reinterpret_cast<const u32x4*>(lo + (first - lead));
     for (uint64_t g = blockIdx.y * 16u + (threadIdx.x >> 4); g < ng; g += 16u * gridDim.y) {
@@ -310,11 +313,17 @@ __global__ __launch_bounds__(256) void k_group_box(const pcr_batch* __restrict__
                 mx[a] = max(mx[a], (uint32_t)__shfl_xor((int)mx[a], m));
             }
         if ((threadIdx.x & 15u) == 0)
-            box[gbase[blockIdx.x] + g] =
+            box[gbase[bi] + g] =
                 make_uint2(mn[0] | (mn[1] << 10) | (mn[2] << 20), mx[0] | (mx[1] << 10) | (mx[2] << 20));
     }
 }
+__global__ __launch_bounds__(256) void k_group_box(const pcr_batch* __restrict__ b, uint32_t nb,
+                                                   const uint32_t* __restrict__ gbase,
+                                                   const uint32_t* __restrict__ lo, uint2* __restrict__ box) {
+    for (uint64_t bi = blockIdx.x; bi < nb; bi += gridDim.x) group_box((uint32_t)bi, b, gbase, lo, box);
+}
 
+constexpr uint32_t kGroupGrid = 1u << 20;
 int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
     const uint32_t nb = c->num_batches;
     if (nb == 0) return PCR_OK;
@@ -342,7 +351,8 @@ int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
     hipStream_t s = ctx->stream;
     const uint32_t rows = (longest + 255) / 256 < 256 ? (longest + 255) / 256 : 256;   // 256 groups or more a workgroup
     PCR_HIP(hipMemcpyAsync(c->d_gbase, base.data(), nb * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    k_group_box<<<dim3(nb, rows), 256, 0, s>>>(c->d_batches, c->d_gbase, c->d_lo, c->d_gbox);
+    k_group_box<<<dim3(nb < kGroupGrid ? nb : kGroupGrid, rows), 256, 0, s>>>(c->d_batches, nb, c->d_gbase, c->d_lo,
+                                                                              c->d_gbox);
     PCR_HIP(hipGetLastError());
     // a sample of the groups: kRows runs of up to kRow, over the whole cloud
     constexpr uint64_t kRows = 16, kRow = 256;

@@ -696,6 +696,7 @@ template <int BLOCK>
 struct GroupList {
     uint32_t open[BLOCK / 64], closed[BLOCK / 64];   // per wave: threads with an open pixel, closed pixels
     uint32_t skipped;                                // points of the hidden groups
+    unsigned long long outside;                      // thread 0: plane bytes of the parts outside the image
     int4 part[BLOCK / 16];                           // batch_range: x0, y0, x1, y1 of 16 groups
     float part_w[BLOCK / 16];                        // and a depth none of their points undercuts
 };
@@ -962,7 +963,8 @@ __device__ __forceinline__ BatchRun next_run(const uint2* __restrict__ box, uint
 
 // One batch of the tiled raster for a cloud with group bounds; `bi` and
 // `level` are workgroup-uniform. Returns the points skipped by the occlusion
-// tests. A batch whose rectangle fits the tile is drawn in one piece. A larger
+// tests; `whole` becomes true when they are all of the item's, every pixel of
+// the batch's rectangle being closed. A batch whose rectangle fits the tile is drawn in one piece. A larger
 // one (a near batch, whose points are spread widely) is drawn in runs of parts
 // of 16 groups: its points are in Morton order, so a part covers about its
 // share of the rectangle, and a run whose rectangle fits the tile is merged
@@ -986,7 +988,7 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
                                                   const uint32_t* __restrict__ hi, const pcr_view& v,
                                                   unsigned long long* __restrict__ fb, unsigned long long* tile,
                                                   uint32_t* natom, bool occl, uint32_t part, uint32_t nparts,
-                                                  const uint2* __restrict__ box, GroupList<BLOCK>& gl) {
+                                                  const uint2* __restrict__ box, GroupList<BLOCK>& gl, bool& whole) {
     pcr_batch h = b[bi];
     if (nparts > 1) {
         const uint32_t f = h.first_point & ~3u;
@@ -1013,6 +1015,7 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
             tests = occl;
             use = fits(tw, th);
             if (tw <= 0) {   // outside the image
+                if (threadIdx.x == 0) gl.outside += 4ull * planes_for_level(level) * h.num_points;
                 if (g >= ng) break;
                 continue;
             }
@@ -1032,6 +1035,7 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
         }
         if (seen == 0) {
             skipped += h.num_points;
+            whole = !parted;
         } else {
             const Decode d = make_decode(level, h.min, h.max);
             const Proj pj = make_proj(v.transform, v.width, v.height);
@@ -1091,7 +1095,7 @@ __global__ __launch_bounds__(BLOCK, !waves_bound(BLOCK, TILE_PIX) ? 1 : KIND == 
     __shared__ uint32_t s_start[kSlices + 1];
     __shared__ GroupList<BLOCK> groups;
     const WorkItems work(st, s_start);
-    if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; s_natom = 0; }
+    if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; s_natom = 0; groups.outside = 0; }
     __syncthreads();
     QueueTake<> q;
     for (;;) {
@@ -1102,30 +1106,30 @@ __global__ __launch_bounds__(BLOCK, !waves_bound(BLOCK, TILE_PIX) ? 1 : KIND == 
         const uint32_t bi = __builtin_amdgcn_readfirstlane(list[slot]);
         const int level = __builtin_amdgcn_readfirstlane(levels[bi]);
         uint32_t skipped;
-        if constexpr (KIND != kNoGroups)
-            skipped = grouped_batch<BLOCK, TILE_PIX, true, KIND == kParts>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0, part,
-                                                     nparts, gbox + gbase[bi], groups);
-        else
+        bool all = false;
+        if constexpr (KIND != kNoGroups) {
+            skipped = grouped_batch<BLOCK, TILE_PIX, true, KIND == kParts>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom,
+                                                                           occl != 0, part, nparts, gbox + gbase[bi],
+                                                                           groups, all);
+        } else {
             skipped = tiled_batch<BLOCK, TILE_PIX, true>(bi, level, b, lo, med, hi, v, fb, tile, &s_natom, occl != 0,
                                                          part, nparts);
+            all = skipped != 0;
+        }
         if (threadIdx.x == 0 && skipped) {
             s_occ_points += skipped;
             s_occ_bytes += 4ull * planes_for_level(level) * skipped;
-            if (part == 0) {   // a batch drawn in parts counts once, by its first
-                pcr_batch h = b[bi];
-                if (nparts > 1) batch_part(h, 0, nparts);
-                s_occ_batches += skipped == h.num_points;
-            }
+            s_occ_batches += all && part == 0;   // a batch drawn in parts counts once, by its first
         }
         __syncthreads();   // s_item and the tile are reused by the next item
     }
     // the loop ends after a barrier that follows every thread's last atomic
     if (threadIdx.x == 0 && s_natom) atomicAdd(&frame_counts(st)->atomics, (unsigned long long)s_natom);
-    if (threadIdx.x == 0 && s_occ_points) {
+    if (threadIdx.x == 0 && s_occ_bytes + groups.outside) {
         FrameCounts* c = frame_counts(st);
         atomicAdd(&c->occluded_batches, s_occ_batches);
         atomicAdd(&c->occluded_points, s_occ_points);
-        atomicAdd(&c->occluded_bytes, s_occ_bytes);
+        atomicAdd(&c->occluded_bytes, s_occ_bytes + groups.outside);
     }
 }
 
@@ -1467,9 +1471,10 @@ __global__ __launch_bounds__(BLOCK, TILE_PIX <= 2048 ? 6 : 1) void k_mv_raster_t
                     continue;
                 }
             }
+            bool all;   // this launch reports no counts
             if (gbox)
                 grouped_batch<BLOCK, TILE_PIX, false, true>(bi, lv, b, lo, med, hi, views[vi], fbs[vi], tile, &s_natom,
-                                                      occl != 0, part, nparts, gbox + gbase[bi], groups[0]);
+                                                            occl != 0, part, nparts, gbox + gbase[bi], groups[0], all);
             else
                 tiled_batch<BLOCK, TILE_PIX, false, true>(bi, lv, b, lo, med, hi, views[vi], fbs[vi], tile, &s_natom,
                                                       occl != 0, part, nparts, &ra);
@@ -1758,6 +1763,7 @@ template <int BLOCK>
 struct HqsGroups {
     uint32_t closed[2][BLOCK / 64];   // per view of a pair and wave
     uint32_t skipped;                 // points of the groups left out
+    unsigned long long outside;       // thread 0: bytes of the parts outside the image
     int4 part[BLOCK / 16];            // batch_parts()
     float part_w[BLOCK / 16];
     __device__ __forceinline__ bool many(int view, int n) const {
@@ -1848,16 +1854,17 @@ __device__ __forceinline__ void hqs_sums_flush(const unsigned long long* tacc, u
     }
 }
 
-// Returns the points skipped by the occlusion test (0 if the batch drew).
+// Returns the points skipped by the occlusion tests; `whole` as in
+// grouped_batch().
 template <int BLOCK, int TILE_PIX, int PASS, bool NT>
 __device__ __forceinline__ uint32_t hqs_tiled_batch(uint32_t bi, int level, const pcr_batch* __restrict__ b,
                                                 const uint32_t* __restrict__ lo, const uint32_t* __restrict__ med,
                                                 const uint32_t* __restrict__ hi, const uint32_t* __restrict__ rgba,
                                                 const pcr_view& v, uint32_t* __restrict__ depth,
                                                 uint32_t* __restrict__ acc, uint32_t* tdepth,
-                                                unsigned long long* tacc, bool occl, uint32_t part = 0,
-                                                uint32_t nparts = 1, const uint2* __restrict__ box = nullptr,
-                                                HqsGroups<BLOCK>* hg = nullptr) {
+                                                unsigned long long* tacc, bool occl, uint32_t part,
+                                                uint32_t nparts, const uint2* __restrict__ box,
+                                                HqsGroups<BLOCK>* hg, bool& whole) {
     const pcr_batch h = b[bi];
     pcr_batch hp = h;   // the points this item draws; the tile and band choices follow the whole batch
     if (nparts > 1) {
@@ -1876,8 +1883,10 @@ __device__ __forceinline__ uint32_t hqs_tiled_batch(uint32_t bi, int level, cons
     // pass 1: behind every depth already drawn over the rectangle; pass 2:
     // behind 1.01x every final depth there (rect_open)
     if (occl && wlo > 0.0f && tw >= 2 && tw * th <= kOcclusionMaxPix &&
-        !rect_open<BLOCK, PASS == 0 ? 1 : 2>(depth, v.width, x0, y0, tw, tw * th, wlo))
+        !rect_open<BLOCK, PASS == 0 ? 1 : 2>(depth, v.width, x0, y0, tw, tw * th, wlo)) {
+        whole = true;
         return hp.num_points;
+    }
     constexpr int cap = HqsTile<PASS, TILE_PIX>::kCap;
     // one-column rectangles draw directly, as in tiled_batch (tw >= 2 keeps
     // the row split's ceil(2^32 / tw) within 32 bits)
@@ -1894,7 +1903,10 @@ __device__ __forceinline__ uint32_t hqs_tiled_batch(uint32_t bi, int level, cons
         for (uint32_t g = 0; g < ng;) {
             const uint32_t gr = g;
             const BatchRun r = next_run<BLOCK, cap>(box, g, ng, h, first, np, lead, level, v, wnear, *hg);
-            if (r.tw <= 0) continue;   // outside the image
+            if (r.tw <= 0) {   // outside the image
+                if (threadIdx.x == 0) hg->outside += (4ull * planes_for_level(level) + (PASS == 1 ? 4ull : 0ull)) * r.num;
+                continue;
+            }
             hp.first_point = r.first;
             hp.num_points = r.num;
             if (!run_fits<cap>(r.tw, r.th)) {
@@ -2277,7 +2289,7 @@ void k_hqs_tiled(const pcr_batch* __restrict__ b,
     const WorkItems work(st, s_start);
     __shared__ uint32_t s_occ_batches;
     __shared__ unsigned long long s_occ_points, s_occ_bytes;   // what the occlusion test skipped
-    if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; }
+    if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; hg.outside = 0; }
     __syncthreads();
     QueueTake<> q;
     for (;;) {
@@ -2287,27 +2299,24 @@ void k_hqs_tiled(const pcr_batch* __restrict__ b,
         const uint64_t slot = work.slot(item, s_start, nb, part, nparts);
         const uint32_t bi = __builtin_amdgcn_readfirstlane(list[slot]);
         const int level = __builtin_amdgcn_readfirstlane(levels[bi]);
+        bool all = false;
         const uint32_t skipped = hqs_tiled_batch<BLOCK, TILE_PIX, PASS, true>(bi, level, b, lo, med, hi, rgba, v,
                                                                               depth, acc, tile.depth, tile.acc,
                                                                               occl != 0, part, nparts,
                                                                               gbox ? gbox + gbase[bi] : nullptr,
-                                                                              &hg);
+                                                                              &hg, all);
         if (threadIdx.x == 0 && skipped) {
             s_occ_points += skipped;
             s_occ_bytes += (4ull * planes_for_level(level) + (PASS == 1 ? 4ull : 0ull)) * skipped;
-            if (part == 0) {   // as in k_raster_tiled
-                pcr_batch h = b[bi];
-                if (nparts > 1) batch_part(h, 0, nparts);
-                s_occ_batches += skipped == h.num_points;
-            }
+            s_occ_batches += all && part == 0;   // as in k_raster_tiled
         }
         __syncthreads();   // s_item and the tile are reused by the next item
     }
-    if (threadIdx.x == 0 && s_occ_points) {
+    if (threadIdx.x == 0 && s_occ_bytes + hg.outside) {
         FrameCounts* c = frame_counts(st);
         atomicAdd(&c->occluded_batches, s_occ_batches);
         atomicAdd(&c->occluded_points, s_occ_points);
-        atomicAdd(&c->occluded_bytes, s_occ_bytes);
+        atomicAdd(&c->occluded_bytes, s_occ_bytes + hg.outside);
     }
 }
 
@@ -2431,10 +2440,10 @@ __global__ __launch_bounds__(BLOCK, PASS == 1 && TILE_PIX <= 2048 ? 4 : 1) void 
                     }
                 }
             }
+            bool all;   // this launch reports no counts
             hqs_tiled_batch<BLOCK, TILE_PIX, PASS, false>(bi, lv, b, lo, med, hi, rgba, views[vi], depths[vi],
                                                            accs[vi], tile.depth, tile.acc, occl != 0, part, nparts,
-                                                           gbox ? gbox + gbase[bi] : nullptr,
-                                                           &hg);
+                                                           gbox ? gbox + gbase[bi] : nullptr, &hg, all);
             __syncthreads();   // the tile is reused by the next view
             k++;
         }

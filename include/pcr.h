@@ -165,15 +165,19 @@ typedef struct pcr_stats {
     float    ms_clear;
     uint64_t batches_occluded;     /* tiled LAS2/NODES/HQS/NODES_HQS draws skipped
                                       because every pixel of the batch's screen
-                                      rectangle already held a nearer point (hqs:
-                                      both passes, a batch per pass)            */
+                                      rectangle (one that fits the tile) already
+                                      held a nearer point (hqs: both passes, a
+                                      batch per pass; of a batch that several
+                                      workgroups share its first part counts)   */
     uint64_t points_occluded;      /* the points of those batches, and of the 64-point
                                       groups left out of others for the same reason */
     uint64_t bytes_occluded;       /* the plane bytes (hqs pass 2: and colour
-                                      bytes) those points did not take; the
-                                      raster's bytes are bytes_algorithmic minus
-                                      these (hqs: twice the planes plus the colour
-                                      of the drawn points, minus these)          */
+                                      bytes) of the drawn batches that were not
+                                      read: those of points_occluded, and of parts
+                                      of large batches that lie outside the image;
+                                      the raster's bytes are bytes_algorithmic
+                                      minus these (hqs: twice the planes plus the
+                                      colour of the drawn points, minus these)  */
     uint64_t atomics_issued;       /* 64-bit framebuffer atomicMins issued (LAS,
                                       LAS2, NODES): those whose compare load found
                                       a larger key                                */

@@ -1022,7 +1022,7 @@ __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const 
         } else {
             use = use && fits(tw, th);
         }
-        const int n = tw * th;
+        const int n = use ? tw * th : 0;   // a part without a bound is over 2^20 pixels wide and high
         const uint32_t magic = use ? row_magic(tw) : 0u;
         int seen = 1;
         if (use) {

@@ -352,6 +352,18 @@ int pcr_cloud_destroy(pcr_cloud* c) {
     return PCR_OK;
 }
 
+// For tests: leaves a cloud as it is where the memory for its group bounds was
+// not there, so that the paths of such clouds can be compared. No plan or
+// captured frame of the cloud may exist.
+extern "C" int pcr_test_drop_group_bounds(pcr_cloud* c) {
+    PCR_CHECK(c, "test_drop_group_bounds: null cloud");
+    PCR_HIP(hipDeviceSynchronize());
+    PCR_HIP(hipFree(c->d_gbox));
+    c->d_gbox = nullptr;
+    c->d_gbase = nullptr;
+    return PCR_OK;
+}
+
 // ------------------------------------------------------------ framebuffers
 int pcr_fb_create(pcr_ctx* ctx, int width, int height, int kind, pcr_fb** out) {
     PCR_CHECK(ctx && out, "fb_create: null argument");

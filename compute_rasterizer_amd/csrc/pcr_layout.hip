@@ -323,6 +323,45 @@ __global__ __launch_bounds__(256) void k_group_box(const pcr_batch* __restrict__
     for (uint64_t bi = blockIdx.x; bi < nb; bi += gridDim.x) group_box((uint32_t)bi, b, gbase, lo, box);
 }
 
+// How far the points of a group lie apart within their batch, as a share of
+// the batch's longest edge: the mean over every total / 1024-th group. One
+// workgroup, a thread a group: finding its batch, a chain of some 17 loads, is
+// what it takes.
+__global__ __launch_bounds__(1024) void k_group_spread(const pcr_batch* __restrict__ b, uint32_t nb,
+                                                       const uint32_t* __restrict__ gbase,
+                                                       const uint2* __restrict__ box, uint64_t total,
+                                                       float* __restrict__ mean) {
+    __shared__ float s_sum[16];
+    const uint32_t n = (uint32_t)(total < 1024 ? total : 1024);
+    float sum = 0.0f;
+    if (threadIdx.x < n) {
+        const uint32_t g = (uint32_t)(total * threadIdx.x / n);
+        uint32_t lo = 0, hi = nb;   // gbase[lo] <= g, and gbase[hi] > g or hi == nb
+        while (hi - lo > 1) {
+            const uint32_t mid = lo + (hi - lo) / 2;
+            if (gbase[mid] <= g) lo = mid;
+            else hi = mid;
+        }
+        float whole = 0.0f, part = 0.0f;
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            const float e = b[lo].max[a] - b[lo].min[a];
+            const int d = (int)((box[g].y >> (10 * a)) & 1023u) - (int)((box[g].x >> (10 * a)) & 1023u);
+            whole = fmaxf(whole, e);
+            part = fmaxf(part, e * (float)max(d, 0) * (1.0f / 1024.0f));
+        }
+        if (whole > 0.0f) sum = part / whole;
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) sum += __shfl_xor(sum, m);
+    if (__lane_id() == 0) s_sum[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) sum += s_sum[w];
+        *mean = sum / (float)n;
+    }
+}
+
 constexpr uint32_t kGroupGrid = 1u << 20;
 int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
     const uint32_t nb = c->num_batches;
@@ -342,7 +381,7 @@ int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
     }
     if (total == 0 || total >= (1ull << 32)) return PCR_OK;
     uint2* box = nullptr;
-    if (hipMalloc(&box, total * sizeof(uint2) + nb * sizeof(uint32_t)) != hipSuccess) {
+    if (hipMalloc(&box, total * sizeof(uint2) + (nb + 1ull) * sizeof(uint32_t)) != hipSuccess) {
         (void)hipGetLastError();
         return PCR_OK;
     }
@@ -354,31 +393,17 @@ int cloud_build_groups(pcr_ctx* ctx, pcr_cloud* c) {
     k_group_box<<<dim3(nb < kGroupGrid ? nb : kGroupGrid, rows), 256, 0, s>>>(c->d_batches, nb, c->d_gbase, c->d_lo,
                                                                               c->d_gbox);
     PCR_HIP(hipGetLastError());
-    // a sample of the groups: kRows runs of up to kRow, over the whole cloud
-    constexpr uint64_t kRows = 16, kRow = 256;
-    const uint64_t rows_n = total < kRows * kRow ? 1 : kRows, row = total < kRows * kRow ? total : kRow;
-    std::vector<uint2> sample(rows_n * row);
-    PCR_HIP(hipMemcpy2DAsync(sample.data(), row * sizeof(uint2), c->d_gbox, total / rows_n * sizeof(uint2),
-                             row * sizeof(uint2), rows_n, hipMemcpyDeviceToHost, s));
+    // its result lies behind the group bases
+    k_group_spread<<<1, 1024, 0, s>>>(c->d_batches, nb, c->d_gbase, c->d_gbox, total, reinterpret_cast<float*>(c->d_gbase + nb));
+    PCR_HIP(hipGetLastError());
+    float spread = 0;
+    PCR_HIP(hipMemcpyAsync(&spread, c->d_gbase + nb, sizeof(float), hipMemcpyDeviceToHost, s));
     PCR_HIP(hipStreamSynchronize(s));
-    c->device_bytes += total * sizeof(uint2) + nb * sizeof(uint32_t);
-    double spread = 0;
-    for (uint64_t k = 0; k < sample.size(); k++) {
-        const uint32_t g = (uint32_t)(k / row * (total / rows_n) + k % row);
-        const pcr_batch& h = c->h_batches[std::upper_bound(base.begin(), base.end(), g) - base.begin() - 1];
-        float whole = 0, part = 0;
-        for (int a = 0; a < 3; a++) {
-            const float e = h.max[a] - h.min[a];
-            const int n = (int)((sample[k].y >> (10 * a)) & 1023u) - (int)((sample[k].x >> (10 * a)) & 1023u);
-            whole = std::max(whole, e);
-            part = std::max(part, e * (float)std::max(n, 0) / 1024.0f);
-        }
-        spread += whole > 0.0f ? part / whole : 0.0;
-    }
+    c->device_bytes += total * sizeof(uint2) + (nb + 1) * sizeof(uint32_t);
     // 0.98 for points in a random order, 0.03 to 0.17 for sorted ones and for
     // flight lines; 0.57 and 0.75 (a city, each building's points together)
     // still gain from the parts
-    c->unsorted = spread > 0.8 * (double)sample.size();
+    c->unsorted = spread > 0.8f;
     std::nth_element(edge.begin(), edge.begin() + nb / 2, edge.end());
     c->batch_edge = edge[nb / 2];
     return PCR_OK;

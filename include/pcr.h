@@ -112,7 +112,12 @@ typedef struct pcr_render_params {
     int32_t  lod_rule;          /* pcr_lod_rule (PCR_MODE_NODES only)              */
     float    lod_px;            /* LOD screen-space error threshold in pixels      */
     uint32_t background;        /* RGBA8 written where nothing was drawn           */
-    int32_t  block_size;        /* raster workgroup size: 0 = default (256)        */
+    int32_t  block_size;        /* raster workgroup size: 0 = default (256), else
+                                   64/128/256/512. LAS: 0 merges the points of a
+                                   batch in a 2048-pixel tile, as LAS2 does, without
+                                   occlusion tests; a size, and any LAS draw of
+                                   pcr_render_static, draws point by point (0 there:
+                                   128). The keys are the same                    */
     int32_t  clear_before;      /* 1: clear the framebuffer before rasterising     */
     int32_t  time_stages;       /* 1: record HIP events around each stage; 2:
                                    around the raster stage only (two events a
@@ -120,7 +125,7 @@ typedef struct pcr_render_params {
     int32_t  tile_px;           /* LAS2/NODES/HQS/NODES_HQS: batches (or parts of
                                    them) whose screen rectangle fits in this many
                                    pixels merge in an LDS tile first (0 = off, else
-                                   1024/2048/4096);
+                                   1024/2048/4096; LAS takes no notice of it);
                                    same result. For hqs it also merges the colour
                                    sums, which is what makes dense views fast    */
     uint32_t batch_begin;       /* draw batches [batch_begin, batch_end) only;     */
@@ -513,6 +518,9 @@ int pcr_selftest_divide(pcr_ctx* ctx, const float* num_x, const float* num_y, co
  *                   batch's last point + 1 rounded up to 4
  *   keys_dev        view->width * view->height uint64 keys, 16-byte aligned
  *   params          time_stages must be 0; mode LAS, LAS2 or NODES
+ *                   (no group bounds are at hand here: batches are drawn
+ *                   whole, LAS point by point, one list of batches in place
+ *                   of pcr_render's slices by depth; the keys are the same)
  *   stream          a hipStream_t of the current device (NULL = null stream) */
 #define PCR_STATIC_MAX_BATCHES 262144u
 int pcr_render_static(const pcr_batch* batches_dev, uint32_t nbatches, const uint32_t* lo_dev,

@@ -109,8 +109,7 @@ def frame_counters(ctx, cloud, views, prm):
         planes = st.bytes_algorithmic - 64 * st.batches_total
         out.append({"drawn_batches": drawn, "points_drawn": st.points_drawn, "points_occluded": st.points_occluded,
                     # raster, algorithmic: headers of the frustum-visible batches, a level byte each, and the
-                    # planes their precision levels need; read: less the planes of batches the occlusion test
-                    # skipped
+                    # planes their precision levels need; read: less the planes of what the raster left out
                     "raster_bytes": 64 * drawn + drawn + planes,
                     "raster_bytes_read": 64 * drawn + drawn + planes - st.bytes_occluded,
                     "frame_bytes": st.bytes_algorithmic + FRAME_BYTES_PER_PIXEL * v.width * v.height,
@@ -151,7 +150,7 @@ def second_flythrough_leg(ctx, cloud, cfg, n_points, width, height, frames, tile
             "raster_ms_mean": round(float(raster.mean()), 4),
             "points_drawn_mean": int(np.mean([cnt[i]["points_drawn"] for i in idx])),
             "points_occluded_mean": int(np.mean([cnt[i]["points_occluded"] for i in idx])),
-            "raster_GBs": round(sum(cnt[i]["raster_bytes"] for i in idx) / (raster.sum() / 1e3) / 1e9, 1)}
+            "raster_GBs": round(sum(cnt[i]["raster_bytes_read"] for i in idx) / (raster.sum() / 1e3) / 1e9, 1)}
 
 
 def overview_leg(ctx, cloud, cfg, n_points, width, height, frames, tile):
@@ -169,10 +168,11 @@ def overview_leg(ctx, cloud, cfg, n_points, width, height, frames, tile):
             "batches_drawn": int(cnt["drawn_batches"]), "points_drawn": int(cnt["points_drawn"]),
             "points_occluded": int(cnt["points_occluded"]), "pixels_visible": int(cnt["pixels_visible"]),
             "atomics_issued": int(cnt["atomics"]), "levels": cnt["levels"],
-            "roofline_raster": {"achieved": round(cnt["raster_bytes"] / (raster.mean() / 1e3) / 1e9, 1),
+            "roofline_raster": {"achieved": round(cnt["raster_bytes_read"] / (raster.mean() / 1e3) / 1e9, 1),
                                 "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                                "frac": round(cnt["raster_bytes"] / (raster.mean() / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
-                                "bytes_per_launch": int(cnt["raster_bytes"])}}
+                                "frac": round(cnt["raster_bytes_read"] / (raster.mean() / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
+                                "bytes_per_launch": int(cnt["raster_bytes"]),
+                                "bytes_read_per_launch": int(cnt["raster_bytes_read"])}}
 
 
 MV_SIZES = [(256, 256), (640, 480), (1280, 720), (1920, 1080), (2560, 1440)]
@@ -772,7 +772,8 @@ def main():
     frame_ms = ft[:, 4].astype(np.float64)   # raster end to raster end
     frame_ms = frame_ms[frame_ms > 0]
     mean = lambda key: float(np.mean([cnt[i][key] for i in idx]))  # noqa: E731
-    achieved = sum(cnt[i]["raster_bytes"] for i in idx) / (raster_ms.sum() / 1e3) / 1e9
+    # the bytes the raster reads: planes of hidden groups and of parts outside the image are not among them
+    achieved = sum(cnt[i]["raster_bytes_read"] for i in idx) / (raster_ms.sum() / 1e3) / 1e9
     frame_gbs = mean("frame_bytes") / (frame_ms.mean() / 1e3) / 1e9
     value = info.num_points * K / wall / 1e9
     kernel = ("k_raster_tiled<%d,%d>" % (args.block if args.block in (128, 256) else 256, args.tile_px)
@@ -794,6 +795,7 @@ def main():
         roof["traffic"] = int(prof["traffic_bytes_per_launch"])
         roof["traffic_over_algorithmic"] = round(prof["traffic_bytes_per_launch"] /
                                                  prof["algorithmic_bytes_per_launch"], 3)
+        roof["traffic_over_read"] = round(prof["traffic_bytes_per_launch"] / prof["read_bytes_per_launch"], 3)
         # issue-side bound beside the HBM fraction, from the same profiled launches
         for k in ("valu_busy_frac", "tcc_hit_frac"):
             if k in prof:

@@ -516,11 +516,15 @@ int pcr_render(pcr_ctx* ctx, pcr_cloud* cloud, const pcr_view* view, const pcr_r
         case PCR_MODE_PLAIN16: rc = launch_raster_points16(s, cloud, *view, fb->d_keys); break;
         case PCR_MODE_LAS:
             // The keys are the same on either path. Point by point the frame is
-            // bound by one atomic request per point (100M-point terrain, 21.9M
-            // points drawn: 181 us); merged in tiles it takes 99. The occlusion
-            // tests stay off: this mode reports none, and over a terrain they
-            // cost more (128) than they leave out. A chosen workgroup size asks
-            // for the point-by-point kernel of that size.
+            // bound by one atomic request per point; merged in tiles (us, point
+            // by point and in tiles): 100M-point terrain from 100 m 181 and 97,
+            // from above 1,228 and 201, 1e9-point city 1,025 and 350, 6,290 and
+            // 1,295, 1M points 98 and 35, 50M unsorted 775 and 751. Half-sorted
+            // points from above can lose (10M at 2560x1440: 189 and 228). The
+            // occlusion tests stay off: this mode reports none. With them (mode
+            // LAS2) up to 100M points take 3 to 12 % more, 1e9 points of a city
+            // 272 and 961 for 350 and 1,295. A chosen workgroup size asks for
+            // the point-by-point kernel of that size.
             rc = cloud->d_gbox && block == 0 ? launch_raster_tiled(s, cloud, *view, 2048, 0, st, fb->d_keys, false)
                                              : launch_raster_batched(s, cloud, *view, 1, block ? block : 128, st, fb->d_keys);
             break;

@@ -706,8 +706,10 @@ struct GroupList {
 // it fails lds_min's first read. Returns 0 when no pixel may take a point at depth wlo
 // or beyond (the batch is hidden; rect_open has the reasons), 1 when some may,
 // 2 when also at least a quarter of them may not. (The test of the groups
-// then leaves out enough to pay: from half on, the overview below takes 1,160
-// us for 1,135, from three quarters on 1,245.)
+// then leaves out enough to pay. From a half and from three quarters on, a
+// 1e9-point city from above takes 985 and 1,058 us for 963, a 1e9-point terrain
+// on 640x400 pixels 1,163 and 1,250 for 1,018; a 100M-point terrain from 100 m
+// 104 and 102 for 108.)
 // Ends in a barrier.
 template <int BLOCK>
 __device__ __forceinline__ int tile_preload(unsigned long long* tile, const unsigned long long* __restrict__ fb, int x0,
@@ -976,12 +978,13 @@ __device__ __forceinline__ BatchRun next_run(const uint2* __restrict__ box, uint
 //
 // Measured, with the near-first slices: the 1e9-point city from 100 m
 // (1920x1080, 19,494 batches drawn) 419 -> 333 us a frame, with 2.9 -> 0.8 M
-// atomic requests and 57% of the points left out (19% before); from above
-// (96,853 batches) 1,284 -> 1,135 us; 1,821 nodes of an octree 261 -> 236 us.
-// The slices and the group test alone gave 410, 1,020 and 262: the registers
-// of the parts cost the overview a fifth wave per SIMD's worth of latency. A
-// kernel of its own for the large batches, before this one, was slower (443
-// us): its waits for memory no longer overlap the other batches' arithmetic.
+// atomic requests and half of the points left out (16% before), 272 since the
+// counters have lines of their own; 1,821 nodes of an octree 261 -> 236, and
+// 222. The slices and the group test without the parts gave 410 and 262 there:
+// the parts are for near batches. Views from far outside have none and run
+// without them (whole_batches). A kernel of its own for the large batches,
+// before this one, was slower (443 us for 333): its waits for memory no longer
+// overlap the other batches' arithmetic.
 template <int BLOCK, int TILE_PIX, bool NT, bool PARTS>
 __device__ __forceinline__ uint32_t grouped_batch(uint32_t bi, int level, const pcr_batch* __restrict__ b,
                                                   const uint32_t* __restrict__ lo, const uint32_t* __restrict__ med,
@@ -1758,7 +1761,10 @@ __device__ __forceinline__ void hqs_sums_preload(uint32_t* tdepth, unsigned long
 // Group test of pass 2: the final depths are known, so 0.6 of the groups of a
 // dense cloud are behind them. Tests the group's rectangle against
 // a view's tile; the reasoning is rect_open's (kind 2).
-constexpr uint32_t kHqsGateDiv = 8;   // from this share of closed pixels on the groups are tested
+// The groups are tested from an eighth of closed pixels on. The line hardly
+// matters (from a half to a sixteenth all frames within 1 %); without the test
+// the stereo frame of a 1e9-point city takes 1,880 us for 1,805.
+constexpr uint32_t kHqsGateDiv = 8;
 template <int BLOCK>
 struct HqsGroups {
     uint32_t closed[2][BLOCK / 64];   // per view of a pair and wave

@@ -22,20 +22,24 @@ __host__ __device__ inline uint32_t groups_of(uint32_t first, uint32_t n) {
 // workgroups and all of them two parts can leave the chip idle half the time
 // (977 batches, 1,536 workgroups: 1,954 halves, two rounds), so there the
 // number of parts with the fewest rounds is taken: 10M points from above 84 us
-// in halves, 78 in thirds; unsorted 315 and 300.
+// in halves, 78 in thirds; unsorted 315 and 300. Batches of one length need
+// that (`even`). The raster of octree nodes, whose lengths differ, fills its
+// second round by itself, and the smaller parts cost it more flushes (50M
+// points 114 us in halves, 119 in thirds); the hqs passes over nodes gain (40M
+// points 275 and 240).
 constexpr uint32_t kMaxParts = 16;
 struct ItemSplit {
     uint32_t whole, nsplit, nparts, items;
     static __host__ __device__ inline uint32_t rounds(uint32_t count, uint32_t groups, uint32_t parts) {
         return (count * parts + groups - 1) / groups;
     }
-    __host__ __device__ inline void split(uint32_t count, uint32_t groups) {
+    __host__ __device__ inline void split(uint32_t count, uint32_t groups, bool even = true) {
         nsplit = count < groups ? count : groups;
         whole = count - nsplit;
         nparts = 2u;
         if (count && count * 2u <= groups) {
             nparts = groups / count < kMaxParts ? groups / count : kMaxParts;
-        } else if (count < groups) {   // the fewest rounds of the workgroups, in batches
+        } else if (even && count < groups) {   // the fewest rounds of the workgroups, in batches
             for (uint32_t p = 3; p <= 4; p++)
                 if (rounds(count, groups, p) * nparts < rounds(count, groups, nparts) * p) nparts = p;
         }

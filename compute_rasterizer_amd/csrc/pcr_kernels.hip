@@ -637,7 +637,7 @@ __device__ __forceinline__ RectInfo uniform_rect(const RectInfo& s) {
 struct WorkItems : ItemSplit {
     // `start` (LDS, kSlices + 1 words) takes the first item of each slice;
     // every thread of the workgroup constructs it (it ends in a barrier)
-    __device__ __forceinline__ WorkItems(const FrameState* st, uint32_t* start) {
+    __device__ __forceinline__ WorkItems(const FrameState* st, uint32_t* start, bool even = true) {
         if (threadIdx.x == 0) {
             uint32_t n = 0;
             for (uint32_t k = 0; k < kSlices; k++) {
@@ -647,7 +647,7 @@ struct WorkItems : ItemSplit {
             start[kSlices] = n;
         }
         __syncthreads();
-        split(__builtin_amdgcn_readfirstlane(start[kSlices]), gridDim.x);
+        split(__builtin_amdgcn_readfirstlane(start[kSlices]), gridDim.x, even);
     }
     // place in a list of nb entries a slice, part and number of parts of an item
     __device__ __forceinline__ uint64_t slot(uint32_t item, const uint32_t* start, uint32_t nb, uint32_t& part,
@@ -1091,13 +1091,13 @@ __global__ __launch_bounds__(BLOCK, !waves_bound(BLOCK, TILE_PIX) ? 1 : KIND == 
                                                         const uint32_t* __restrict__ hi, pcr_view v,
                                                         unsigned long long* __restrict__ fb, int occl,
                                                         uint32_t nb, const uint2* __restrict__ gbox,
-                                                        const uint32_t* __restrict__ gbase) {
+                                                        const uint32_t* __restrict__ gbase, int even) {
     __shared__ unsigned long long tile[TILE_PIX];
     __shared__ uint32_t s_item, s_occ_batches, s_natom;   // s_natom: framebuffer atomics issued
     __shared__ unsigned long long s_occ_points, s_occ_bytes;   // what the occlusion test skipped
     __shared__ uint32_t s_start[kSlices + 1];
     __shared__ GroupList<BLOCK> groups;
-    const WorkItems work(st, s_start);
+    const WorkItems work(st, s_start, even != 0);
     if (threadIdx.x == 0) { s_occ_batches = 0; s_occ_points = 0; s_occ_bytes = 0; s_natom = 0; groups.outside = 0; }
     __syncthreads();
     QueueTake<> q;
@@ -1151,7 +1151,8 @@ static void tiled_grid(hipStream_t s, const pcr_cloud* c, const pcr_view& v, Fra
     if (grid > (uint64_t)c->num_batches * kMaxParts) grid = (uint64_t)c->num_batches * kMaxParts;
     k_raster_tiled<BLOCK, TILE_PIX, KIND><<<(int)grid, BLOCK, 0, s>>>(c->d_batches, c->d_levels, c->d_list, st, c->d_lo,
                                                                c->d_med, c->d_hi, v, fb, occl ? 1 : 0,
-                                                               c->num_batches, c->d_gbox, c->d_gbase);
+                                                               c->num_batches, c->d_gbox, c->d_gbase,
+                                                               c->num_levels == 0 ? 1 : 0);
 }
 
 // Whether k_raster_tiled draws the view's batches whole (kWhole): the cloud's
